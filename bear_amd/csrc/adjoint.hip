@@ -293,14 +293,16 @@ template <int NS>
 __device__ __forceinline__ void emitLevel(double* __restrict__ out, int lane, double kbar,
                                           const double* __restrict__ t, double tbar, double zbar,
                                           double scaling) {
-  double x[NS + 4];
+  constexpr int K = int(adjointSlots(NS, false, false));
+  double x[K];
 #pragma unroll
   for (int s = 0; s < NS; ++s) x[s] = kbar * t[s * kWave];
   x[NS] = tbar;
   x[NS + 1] = zbar;
   x[NS + 2] = scaling;
-  x[NS + 3] = 0.0;
-  emitSums<NS + 4>(out, lane, x, 0, NS + 4);
+#pragma unroll
+  for (int s = NS + 3; s < K; ++s) x[s] = 0.0;
+  emitSums<K>(out, lane, x, 0, K);
 }
 
 // Forward sweep into scratch = [grid][levels][2][64], then the backward
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(kWave) void emissionAdjointKernel(
     const double* __restrict__ wavenumber, const double* __restrict__ tables, size_t stride, Records rec,
     int nb_levels, int n, int tiles, int batch, const double* __restrict__ fbar, double* __restrict__ scratch,
     double* __restrict__ partial) {
-  constexpr int K = NS + 4;
+  constexpr int K = int(adjointSlots(NS, false, false));
   __shared__ double sig[2 * NS * kWave];
   const int L = nb_levels;
   const int lane = int(threadIdx.x);
@@ -560,7 +562,7 @@ __global__ __launch_bounds__(kWave) void opacityAdjointKernel(const double* __re
                                                               const float* __restrict__ keep,
                                                               const double* __restrict__ hminus, int kslots,
                                                               double* __restrict__ partial) {
-  constexpr int KX = NS + 4;
+  constexpr int KX = (NS + 4) / 4 * 4;                              // NS + 1 sums in whole groups of four
   const int K = kslots;                                             // partial row: every level slot
   const int L = nb_levels;
   const int lane = int(threadIdx.x);
@@ -1019,14 +1021,12 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
     raise(kInvalidInput, "the transmission adjoint does not take cloud layers");
   if (batch == 0 || batch > batch_capacity_) raise(kInternal, "adjoint batch larger than the staged records");
   const int NS = int(species_stride_);
-  if (NS != 4 && NS != 8 && NS != 12 && NS != 16) raise(kInvalidInput, "the adjoint takes at most 16 tabulated species");
+  if (species_stride_ > kMaxSlots) raise(kInvalidInput, "the adjoint takes at most 16 tabulated species");
   check(hipSetDevice(device_), "hipSetDevice");
   hipStream_t s = static_cast<hipStream_t>(stream_);
-  // level slots: NS + 4, 8 more for the H- continuum's weights, 16 more for
-  // the cloud models' layer sums
-  const int cloud_slot0 = cloud_models_ > 0 ? NS + (hminus_ ? 12 : 4) : -1;
+  const int cloud_slot0 = cloud_models_ > 0 ? int(adjointCloudSlot(NS, hminus_)) : -1;
   const int n = int(n_points_), L = int(nb_levels_), nb = int(n_bins_),
-            K = NS + (hminus_ ? 12 : 4) + (cloud_models_ > 0 ? 4 * kMaxClouds : 0);
+            K = int(adjointSlots(NS, hminus_, cloud_models_ > 0));
   const int tiles = (n + kWave - 1) / kWave;
   const int grid = int(align8(std::max<size_t>(8, size_t(nb_cus_) * kAdjointWavesPerCu)));
   const int rt_grid = int(align8(std::max<size_t>(8, size_t(nb_cus_) * kRtWavesPerCu)));
@@ -1175,20 +1175,12 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
           win.kept_origin = nu_first / kWave * size_t(L) * kKeptLevel;
           launchBatchSpectrum(ModelKind::transmission, 1, launch, first, keep, nu_first, nu_end - nu_first, reach);
         }
-        switch (NS) {
-#define BEAR_TADJ(NSV)                                                                                             \
-  case NSV:                                                                                                        \
-    launchTransmissionAdjoint<NSV>(dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, tables_, stride_, rayleigh_,  \
-                                   rec, L, n, tiles, win, cb, adj_fbar_, batch_flux_ + first * stride_, keep,     \
-                                   adj_partial_, ranges, r0, r1, nu_per_range, chord_partial, chord_t, reach,     \
-                                   hminus_, K);                                                                   \
-    break;
-          BEAR_TADJ(4)
-          BEAR_TADJ(8)
-          BEAR_TADJ(12)
-          BEAR_TADJ(16)
-#undef BEAR_TADJ
-        }
+        withSlots(species_stride_, [&](auto ns) {
+          launchTransmissionAdjoint<ns>(dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, tables_, stride_, rayleigh_,
+                                        rec, L, n, tiles, win, cb, adj_fbar_, batch_flux_ + first * stride_, keep,
+                                        adj_partial_, ranges, r0, r1, nu_per_range, chord_partial, chord_t, reach,
+                                        hminus_, K);
+        });
         check(hipGetLastError(), "transmission adjoint kernels");
       }
       hipLaunchKernelGGL(chordReduceKernel, dim3(unsigned((P * P + kBlock - 1) / kBlock), unsigned(cb)),
@@ -1198,20 +1190,12 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
                            hipMemcpyDeviceToHost, s),
             "read chord gradients");
     } else {
-    switch (NS) {
-#define BEAR_ADJ(NSV)                                                                                              \
-  case NSV:                                                                                                        \
-    launchAdjoint<NSV>(kept, dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, wavenumber_, wavelength_, tables_,   \
-                       stride_, rec, L, n, tiles, cb, adj_fbar_, adj_intensity_, adj_partial_, hminus_, K,         \
-                       cloud_slot0);                                                                               \
-    break;
-      BEAR_ADJ(4)
-      BEAR_ADJ(8)
-      BEAR_ADJ(12)
-      BEAR_ADJ(16)
-#undef BEAR_ADJ
-    }
-    check(hipGetLastError(), "adjoint kernels");
+      withSlots(species_stride_, [&](auto ns) {
+        launchAdjoint<ns>(kept, dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, wavenumber_, wavelength_, tables_,
+                          stride_, rec, L, n, tiles, cb, adj_fbar_, adj_intensity_, adj_partial_, hminus_, K,
+                          cloud_slot0);
+      });
+      check(hipGetLastError(), "adjoint kernels");
     }
     double* level_out = adj_out_ + first * L * K;
     switch (K) {

@@ -760,39 +760,21 @@ void DeviceEngine::launchBatchSpectrum(ModelKind kind, size_t batch, const Batch
       win.kept_origin = nu_first / kKeptValue * size_t(L) * kKeptLevel;
     }
     const size_t lds = transmissionLds(L, lc.tile, wide);
-    switch (species_stride_) {
-#define BEAR_T(NS)                                                                                                  \
-  case NS:                                                                                                          \
-    launchTransmission<NS>(precision_, dim3(unsigned(lc.grid)), lds, s, tables_, tables_low_, table_base_, stride_, \
-                           rayleigh_, wavelength_, ex, extras, rec, batch_chord_, batch_chord32_, L, n, win,       \
-                           lc.tile, B, lc.group, flux, keep, reach);                                               \
-    break;
-      BEAR_T(4)
-      BEAR_T(8)
-      BEAR_T(12)
-      BEAR_T(16)
-#undef BEAR_T
-      default:
-        raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
-    }
+    const bool launched = withSlots(species_stride_, [&](auto ns) {
+      launchTransmission<ns>(precision_, dim3(unsigned(lc.grid)), lds, s, tables_, tables_low_, table_base_, stride_,
+                             rayleigh_, wavelength_, ex, extras, rec, batch_chord_, batch_chord32_, L, n, win, lc.tile,
+                             B, lc.group, flux, keep, reach);
+    });
+    if (!launched) raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
     check(hipGetLastError(), "transmission batch kernel");
     return;
   }
   const int tiles = (n + lc.block - 1) / lc.block;
-  switch (species_stride_) {
-#define BEAR_E(NS)                                                                                                   \
-  case NS:                                                                                                           \
-    launchEmission<NS>(precision_, dim3(unsigned(lc.grid)), dim3(unsigned(lc.block)), s, wavenumber_, wavelength_,   \
-                       tables_, tables_low_, table_base_, stride_, ex, extras, rec, L, n, tiles, B, flux, keep);    \
-    break;
-    BEAR_E(4)
-    BEAR_E(8)
-    BEAR_E(12)
-    BEAR_E(16)
-#undef BEAR_E
-    default:
-      raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
-  }
+  const bool launched = withSlots(species_stride_, [&](auto ns) {
+    launchEmission<ns>(precision_, dim3(unsigned(lc.grid)), dim3(unsigned(lc.block)), s, wavenumber_, wavelength_,
+                       tables_, tables_low_, table_base_, stride_, ex, extras, rec, L, n, tiles, B, flux, keep);
+  });
+  if (!launched) raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
   check(hipGetLastError(), "emission batch kernel");
 }
 
@@ -893,7 +875,7 @@ void DeviceEngine::evaluateBatch(ModelKind kind, size_t batch) { evaluateBatch(k
 
 void DeviceEngine::evaluateBatch(ModelKind kind, size_t batch, bool staged) {
   if (staged && (!stage_blob_ || batch > stage_capacity_)) raise(kInternal, "device staging not prepared");
-  if (species_stride_ > 16) raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
+  if (species_stride_ > kMaxSlots) raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
   if ((hminus_ || cloud_models_ > 0) && precision_ != TablePrecision::fp64)
     raise(kInvalidInput, "the H- continuum and cloud layers take FP64 tables");
   if (batch == 0 || batch > batch_capacity_) raise(kInternal, "batch larger than the staged records");

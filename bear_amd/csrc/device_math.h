@@ -260,7 +260,7 @@ __device__ __forceinline__ double cloudLayer(const Extras& ex, const double (&cf
 // The same without a register cache, for any number of species: chunks of
 // kChunk slots with every row of a chunk loaded before any is used; weights
 // and densities from each slot's record.
-constexpr int kChunk = 4;
+constexpr int kChunk = int(kSlotChunk);
 
 __device__ __forceinline__ double chunkedKappa(const double* __restrict__ tab, size_t stride,
                                                const LevelSpecies* __restrict__ d, const LevelState& lev,

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "host.h"
@@ -153,6 +154,40 @@ struct alignas(16) LevelSpecies32 {
 enum class TablePrecision : int { fp64 = 0, fp32 = 1, fp16 = 2, bf16 = 3, int16 = 4 };
 inline size_t tableElementBytes(TablePrecision p) {
   return p == TablePrecision::fp64 ? 8 : p == TablePrecision::fp32 ? 4 : 2;
+}
+
+// Stencil slots per level for S tabulated species: one each up to kMaxSlots,
+// for which every register-cached kernel is instantiated at its exact count
+// (a padding slot costs as much as a species: an interpolation and a power
+// of ten per level), beyond that whole chunks of the generic kernel.  Against
+// slots in fours: one point of 2 species (60 levels, 20,000 wavenumbers) 136 ->
+// 114 us, 192 points of 14 (100 levels, 300,000, FP16 tables) 71.6 -> 62.2 ms,
+// 48 transits of 10 (200 levels, 60,000, FP64) 12.4 -> 11.4 ms, the same bits.
+constexpr size_t kMaxSlots = 16, kSlotChunk = 4;
+constexpr size_t stencilSlots(size_t species) {
+  return species == 0 ? 1 : species <= kMaxSlots ? species : (species + kSlotChunk - 1) / kSlotChunk * kSlotChunk;
+}
+
+// f(std::integral_constant<int, NS>) for the slot count ns in 1 .. kMaxSlots;
+// false when it is none of them
+template <int NS = 1, class F>
+bool withSlots(size_t ns, F&& f) {
+  if constexpr (NS > int(kMaxSlots)) {
+    return false;
+  } else {
+    if (ns != size_t(NS)) return withSlots<NS + 1>(ns, f);
+    f(std::integral_constant<int, NS>{});
+    return true;
+  }
+}
+
+// The adjoint's sums per level: NS + 4 (adjoint.hip), 8 more for the H-
+// continuum's weights, 16 more for the cloud models' layer sums from
+// adjointCloudSlot on, in rows of whole groups of four (the wavefront sums
+// take four values at a time)
+constexpr size_t adjointCloudSlot(size_t ns, bool hminus) { return ns + (hminus ? 12 : 4); }
+constexpr size_t adjointSlots(size_t ns, bool hminus, bool clouds) {
+  return (adjointCloudSlot(ns, hminus) + (clouds ? 4 * kMaxClouds : 0) + 3) / 4 * 4;
 }
 
 enum class ModelKind : int { emission = 0, eclipse = 1, transmission = 2 };
@@ -337,7 +372,7 @@ class DeviceEngine {
   void copyBatchSpectrum(ModelKind kind, size_t batch, double* host);  // [batch][N], output units
   // Value and adjoint of the staged batch (emission, FP64 tables): the
   // log-likelihoods (batchLogLikelihood()) and per point dL/d(level
-  // quantities) [batch][levels][speciesStride() + 4]: n dL/dn for the
+  // quantities) [batch][levels][adjointSlots()]: n dL/dn for the
   // effective density n of each stencil slot, the temperature through the table interpolation
   // (recomputing: and through the Planck function), the altitude, the flux
   // scaling (level 0 only; 0 elsewhere), the temperature through the Planck

@@ -302,8 +302,6 @@ void deviceFree(void* p) {
   if (p) (void)hipFree(p);
 }
 
-constexpr size_t kMaxSpecies = 16;                    // register-cached kernels up to 16 species
-
 // scratch's address on `device` (current), resolved once per device
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
@@ -493,8 +491,7 @@ void DeviceEngine::allocateTables(size_t nb_rows, size_t nb_species) {
   }
   // residual rows and the per-species base only; every species passes
   // through an FP64 staging buffer of its own rows (uploadSpeciesRows)
-  const size_t slots = std::max<size_t>(kChunk, (nb_species + kChunk - 1) / kChunk * kChunk);
-  allocateReduced(storage_, nb_rows, slots);
+  allocateReduced(storage_, nb_rows, stencilSlots(nb_species));
 }
 
 void DeviceEngine::uploadSpeciesRows(int slot, size_t first, size_t count, const double* rows) {
@@ -652,9 +649,8 @@ void DeviceEngine::configure(size_t nb_levels, size_t nb_species, bool transmiss
   nb_levels_ = nb_levels;
   nb_species_ = nb_species;
   transmission_ = transmission;
-  species_stride_ = (nb_species + kChunk - 1) / kChunk * kChunk;   // padding entries keep n = 0, row 0
-  if (species_stride_ == 0) species_stride_ = kChunk;
-  if (transmission && species_stride_ > kMaxSpecies)
+  species_stride_ = stencilSlots(nb_species);                        // padding entries keep n = 0, row 0
+  if (transmission && species_stride_ > kMaxSlots)
     raise(kInvalidInput, "the transmission model takes at most 16 tabulated species");
   if (transmission && transmissionLds(nb_levels, 64) > lds_limit_)
     raise(kInvalidInput, "too many levels for the transmission kernel");
@@ -721,25 +717,18 @@ void launchEmission(hipStream_t s, size_t species_stride, int blocks, const doub
                     const double* tables, size_t stride, const Extras& ex, const LevelState* lev,
                     const LevelSpecies* spc, StencilGroups groups, int L, int n, double scaling, SpectrumOut out,
                     double* flux, double* spectrum) {
-  switch (species_stride) {
-#define BEAR_CACHED(NS)                                                                                             \
-  case NS:                                                                                                          \
-    if (hasExtras(ex))                                                                                              \
-      hipLaunchKernelGGL((emissionKernelCached<NS, true>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables,      \
-                         stride, ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);                         \
-    else                                                                                                            \
-      hipLaunchKernelGGL((emissionKernelCached<NS, false>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables,     \
-                         stride, ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);                         \
-    break;
-    BEAR_CACHED(4)
-    BEAR_CACHED(8)
-    BEAR_CACHED(12)
-    BEAR_CACHED(16)
-#undef BEAR_CACHED
-    default:
-      hipLaunchKernelGGL(emissionKernel, dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride, ex, lev,
-                         spc, L, int(species_stride / kChunk), n, scaling, out, flux, spectrum);
-  }
+  const bool cached = withSlots(species_stride, [&](auto ns) {
+    constexpr int NS = ns;
+    if (hasExtras(ex))
+      hipLaunchKernelGGL((emissionKernelCached<NS, true>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride,
+                         ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);
+    else
+      hipLaunchKernelGGL((emissionKernelCached<NS, false>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride,
+                         ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);
+  });
+  if (!cached)
+    hipLaunchKernelGGL(emissionKernel, dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride, ex, lev, spc, L,
+                       int(species_stride / kChunk), n, scaling, out, flux, spectrum);
 }
 }  // namespace
 
@@ -834,26 +823,18 @@ void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius
   const int blocks = (n + tile - 1) / tile;
   const Extras ex = extras();
   beginTimed();
-  switch (species_stride_) {
-#define BEAR_TRANSMISSION(NS)                                                                                       \
-  case NS:                                                                                                          \
-    if (hasExtras(ex))                                                                                              \
-      hipLaunchKernelGGL((transmissionKernel<NS, true>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,  \
-                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,  \
-                         star_radius, buf.flux, spectrum_dev);                                                      \
-    else                                                                                                            \
-      hipLaunchKernelGGL((transmissionKernel<NS, false>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_, \
-                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,  \
-                         star_radius, buf.flux, spectrum_dev);                                                      \
-    break;
-    BEAR_TRANSMISSION(4)
-    BEAR_TRANSMISSION(8)
-    BEAR_TRANSMISSION(12)
-    BEAR_TRANSMISSION(16)
-#undef BEAR_TRANSMISSION
-    default:
-      raise(kInvalidInput, "unsupported number of species for transmission");
-  }
+  const bool launched = withSlots(species_stride_, [&](auto ns) {
+    constexpr int NS = ns;
+    if (hasExtras(ex))
+      hipLaunchKernelGGL((transmissionKernel<NS, true>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
+                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
+                         star_radius, buf.flux, spectrum_dev);
+    else
+      hipLaunchKernelGGL((transmissionKernel<NS, false>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
+                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
+                         star_radius, buf.flux, spectrum_dev);
+  });
+  if (!launched) raise(kInvalidInput, "unsupported number of species for transmission");
   check(hipGetLastError(), "transmission kernel");
   endTimed();
   launchBins(0, 0.0, 0.0, inflation, bins_dev);
