@@ -166,6 +166,20 @@ __global__ __launch_bounds__(kBlock) void fluxAdjointKernel(const uint64_t* __re
   fbar[size_t(m) * stride + i] = acc;
 }
 
+// One layer of the two-angle short characteristics (short_characteristics.cpp:88-114)
+__device__ __forceinline__ void shortCharacteristicsLayer(double tau, double b_prev, double b_next,
+                                                          double& i1, double& i2) {
+  if (tau != 0) {
+    const double r = recip(tau);
+    const double a1 = pow2(tau * (-kLog2E / kMu1));
+    const double q1 = (a1 - 1.0) * (kMu1 * r);
+    i1 = fma(i1, a1, (1.0 + q1) * b_next + (-a1 - q1) * b_prev);
+    const double a2 = pow2(tau * (-kLog2E / kMu2));
+    const double q2 = (a2 - 1.0) * (kMu2 * r);
+    i2 = fma(i2, a2, (1.0 + q2) * b_next + (-a2 - q2) * b_prev);
+  }
+}
+
 // Per slot of one level: the opacity term t_s = n_s sigma_s =
 // 2^(log2 n_s + sum_k w_k v_k), as the forward kernels form it (with
 // kGradientExp the exponential to 1.2e-7, pow2Gradient), and
@@ -188,15 +202,13 @@ __device__ __forceinline__ void slotTerms(const LevelSpecies* __restrict__ d, co
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const bool one = (groups.group1 >> s) & 1u;
-      double x = fma(one ? wb[0] : wa[0], v[s][0], lev.log2_n[s]);
-      x = fma(one ? wb[1] : wa[1], v[s][1], x);
-      x = fma(one ? wb[2] : wa[2], v[s][2], x);
-      x = fma(one ? wb[3] : wa[3], v[s][3], x);
-      double y = (one ? ub[0] : ua[0]) * v[s][0];
-      y = fma(one ? ub[1] : ua[1], v[s][1], y);
-      y = fma(one ? ub[2] : ua[2], v[s][2], y);
-      y = fma(one ? ub[3] : ua[3], v[s][3], y);
+      double x = lev.log2_n[s], y = 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        x = fma(groupWeight<NS>(wa, wb, groups, s, q), v[s][q], x);
+        const double u = groupWeight<NS>(ua, ub, groups, s, q);
+        y = q == 0 ? u * v[s][0] : fma(u, v[s][q], y);
+      }
       f(s, term(x), y);
     }
   } else {
@@ -221,16 +233,12 @@ __device__ __forceinline__ void slotTerms(const LevelSpecies* __restrict__ d, co
 // level processed before this one, the one above, brought new rows; or the
 // first level of the sweep).
 template <int NS>
-__device__ __forceinline__ void levelOpacity(const double* __restrict__ tab, const LevelSpecies* __restrict__ d,
+__device__ __forceinline__ void levelOpacity(const double* __restrict__ tab, unsigned i,
+                                             const LevelSpecies* __restrict__ d,
                                              const LevelSpeciesAdjoint* __restrict__ a, const LevelState& lev,
                                              StencilGroups groups, bool reload, double (&v)[NS][4],
                                              double* __restrict__ t, double& kappa, double& dkdt) {
-  if (reload) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[s][q] = tab[size_t(d[s].block[q]) << 6];
-  }
+  if (reload) loadRows<NS>(tab, i, d, v);
   double k = 0.0, dk = 0.0;
   slotTerms<NS>(d, a, lev, groups, v, [&](int s, double ts, double ys) {
     t[s * kWave] = ts;
@@ -330,7 +338,6 @@ __global__ __launch_bounds__(kWave) void emissionAdjointKernel(
     const LevelSpecies* species = reinterpret_cast<const LevelSpecies*>(r + rec.species);
     const LevelSpeciesAdjoint* extra = reinterpret_cast<const LevelSpeciesAdjoint*>(r + rec.adjoint);
     double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
-    const double* tab = tables + ic;
     const double nu = wavenumber[ic];
     const double b_num = kPlanckC1 * nu * nu * nu;
     const double x_nu = -(6.62606896e-27 * nu * 2.99792458e10 / 1.3806504e-16) * kLog2E;
@@ -339,15 +346,17 @@ __global__ __launch_bounds__(kWave) void emissionAdjointKernel(
     // forward sweep; I_l of angle a at I[l * 2 * 64 + a * 64]
     double* store = scratch + size_t(blockIdx.x) * size_t(L) * 2 * kWave + lane;
     {
-      double k_prev = kappaTerms<NS>(tab, stride, species, levels[0], rec.groups, true, v);
+      loadRows<NS>(tables, unsigned(ic), species, v);
+      double k_prev = kappaFrom<NS>(v, species, levels[0], rec.groups);
       double b_prev = planckAt(b_num, x_nu, levels[0].inv_temperature);
       double z_prev = levels[0].altitude;
       double i1 = b_prev, i2 = b_prev;
       store[0] = i1;
       store[kWave] = i2;
       for (int l = 1; l < L; ++l) {
-        const double k_next = kappaTerms<NS>(tab, stride, species + size_t(l) * NS, levels[l], rec.groups,
-                                             levels[l].reload != 0, v);
+        const LevelSpecies* d = species + size_t(l) * NS;
+        if (levels[l].reload) loadRows<NS>(tables, unsigned(ic), d, v);
+        const double k_next = kappaFrom<NS>(v, d, levels[l], rec.groups);
         const double b_next = planckAt(b_num, x_nu, levels[l].inv_temperature);
         const double z_next = levels[l].altitude;
         shortCharacteristicsLayer((z_next - z_prev) * (k_next + k_prev) * 0.5, b_prev, b_next, i1, i2);
@@ -371,7 +380,7 @@ __global__ __launch_bounds__(kWave) void emissionAdjointKernel(
 
     // backward sweep; level l's cross-sections in LDS half (l & 1)
     double k_hi, dk_hi, b_hi, db_hi;
-    levelOpacity<NS>(tab, species + size_t(L - 1) * NS, extra + size_t(L - 1) * NS, levels[L - 1], rec.groups, true, v,
+    levelOpacity<NS>(tables, unsigned(ic), species + size_t(L - 1) * NS, extra + size_t(L - 1) * NS, levels[L - 1], rec.groups, true, v,
                      my_sig + ((L - 1) & 1) * NS * kWave, k_hi, dk_hi);
     planckAdjoint(b_num, x_nu, levels[L - 1].inv_temperature, b_hi, db_hi);
     double z_hi = levels[L - 1].altitude;
@@ -381,7 +390,7 @@ __global__ __launch_bounds__(kWave) void emissionAdjointKernel(
       const double i1p = below[0];
       const double i2p = below[angle_step];
       double k_lo, dk_lo, b_lo, db_lo;
-      levelOpacity<NS>(tab, species + size_t(l - 1) * NS, extra + size_t(l - 1) * NS, levels[l - 1], rec.groups,
+      levelOpacity<NS>(tables, unsigned(ic), species + size_t(l - 1) * NS, extra + size_t(l - 1) * NS, levels[l - 1], rec.groups,
                        levels[l].reload != 0, v,
                        my_sig + ((l - 1) & 1) * NS * kWave, k_lo, dk_lo);
       planckAdjoint(b_num, x_nu, levels[l - 1].inv_temperature, b_lo, db_lo);
@@ -579,7 +588,6 @@ __global__ __launch_bounds__(kWave) void opacityAdjointKernel(const double* __re
     const LevelSpeciesAdjoint* extra = reinterpret_cast<const LevelSpeciesAdjoint*>(r + rec.adjoint);
     const float* kb = keep + keptAt(win, m, stride, L, ic) + 2 * kKeptValue;
     double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
-    const double* tab = tables + ic;
     double v[NS][4];
     double hm[7];
     if constexpr (HM)
@@ -591,12 +599,7 @@ __global__ __launch_bounds__(kWave) void opacityAdjointKernel(const double* __re
       const double kbar = valid ? kb1 : 0.0;
       const LevelSpecies* d = species + size_t(l) * NS;
       const LevelSpeciesAdjoint* a = extra + size_t(l) * NS;
-      if (l == 0 || levels[l].reload != 0) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[s][q] = tab[size_t(d[s].block[q]) << 6];
-      }
+      if (l == 0 || levels[l].reload != 0) loadRows<NS>(tables, unsigned(ic), d, v);
       kb1 = kb2;
       if (l + 2 < L) kb2 = kb[size_t(l + 2) * kKeptLevel];
       double x[KX];
@@ -1117,7 +1120,11 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
     raise(kInvalidInput, "the H- continuum's gradient needs the kept forward quantities: raise the adjoint memory");
   if (cloud_models_ > 0 && !kept)
     raise(kInvalidInput, "the clouds' gradient needs the kept forward quantities: raise the adjoint memory");
-  const BatchLaunch launch = tuned(transmission ? ModelKind::transmission : ModelKind::emission, chunk);
+  // the emission forward runs in workgroups of 256, the transmission forward
+  // as tuned
+  const BatchLaunch launch = !transmission ? BatchLaunch{256, 256, int(std::min<size_t>(nbItems((n + 255) / 256, int(chunk)), INT32_MAX))}
+                                                   : tuned(kind, chunk);
+  last_launch_ = launch;
   bin_terms.assign(transmission ? batch * P * P : eclipse ? batch * n_bins_ * 2 : 0, 0.0);
   if (profiling_) check(hipEventRecord(static_cast<hipEvent_t>(event_start_), s), "hipEventRecord");
   if (staged) {
@@ -1139,7 +1146,7 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
     double* chord_t = chord_out + size_t(cb) * P * P;
     int* reach = reinterpret_cast<int*>(chord_t + size_t(cb) * P * segmentRows(L));
     launchBatchSpectrum(transmission ? ModelKind::transmission : ModelKind::emission, size_t(cb), launch, first,
-                        windowed ? nullptr : keep, 0, 0, transmission && !windowed ? reach : nullptr);
+                        windowed ? nullptr : keep, 0, 0, transmission && !windowed ? reach : nullptr, true);
     launchBatchRest(kind, size_t(cb), first);
     double* gbar = adj_gbar_ + first * n_bins_;
     double* fscale = eclipse ? adj_fscale_ + first * n_bins_ : gbar;

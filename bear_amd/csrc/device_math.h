@@ -96,12 +96,12 @@ __device__ __forceinline__ double pow2Gradient(double t) {
   return __builtin_amdgcn_ldexp(double(__builtin_amdgcn_exp2f(f)), int(n));
 }
 
-// 1/d for finite non-zero d: hardware estimate and two Newton steps
+// 1/d for finite non-zero d: the hardware estimate r (better than 2^-22) and
+// one third-order step, r (1 + e + e^2) for e = 1 - d r, which leaves e^3
 __device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(fma(-d, r, 1.0), r, r);
-  r = fma(fma(-d, r, 1.0), r, r);
-  return r;
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(fma(e, e, e), r, r);
 }
 
 // Planck function per wavenumber written as c1 nu^3 q / (1 - q),
@@ -127,59 +127,45 @@ __device__ __forceinline__ void starFluxWithDerivative(double nu, double inv_t, 
   d_flux = flux * (-x_nu * kLn2) * inv_t * inv_t * r;
 }
 
-// One layer of the two-angle short characteristics (short_characteristics.cpp:88-114)
-__device__ __forceinline__ void shortCharacteristicsLayer(double tau, double b_prev, double b_next,
-                                                          double& i1, double& i2) {
-  if (tau != 0) {
-    const double r = recip(tau);
-    const double a1 = pow2(tau * (-kLog2E / kMu1));
-    const double q1 = (a1 - 1.0) * (kMu1 * r);
-    i1 = fma(i1, a1, (1.0 + q1) * b_next + (-a1 - q1) * b_prev);
-    const double a2 = pow2(tau * (-kLog2E / kMu2));
-    const double q2 = (a2 - 1.0) * (kMu2 * r);
-    i2 = fma(i2, a2, (1.0 + q2) * b_next + (-a2 - q2) * b_prev);
-  }
-}
-
-// The opacity terms of NH consecutive stencil slots at one level,
+// The opacity terms of NS stencil slots at one level,
 // sum_s 2^(log2 n_s + sum_k w_sk v_sk) with the slots' four table values v
-// kept in registers between levels and all reloaded when `reload` (the
-// level brings new rows for some slot, or the first level)
-// (opacity_species.cpp:277-345, 400-433: the bilinear log10 interpolation in
-// T and log p, times the effective density).  Rows are always valid; a zero
-// density (log2 n = -inf) removes a term exactly.
+// kept in registers between levels and all reloaded when the level brings new
+// rows for some slot (opacity_species.cpp:277-345, 400-433: the bilinear log10
+// interpolation in T and log p, times the effective density).  Rows are always
+// valid; a zero density (kZeroDensityLog2) removes a term exactly.
 // With grouped stencils (StencilGroups) the weights come from the level's two
-// shared sets, group1 holding these NH slots' group bits, and the densities
-// from the level's contiguous copy (NH <= 16, the first NH slots); otherwise
-// both from each slot's record.
-// The two halves are also available apart (loadRows, kappaFrom), so that a
-// kernel can issue the next level's row loads before this level's other
-// work and find them arrived when it needs them.
-template <int NH>
-__device__ __forceinline__ void loadRows(const double* __restrict__ tab, const LevelSpecies* __restrict__ d,
-                                         double (&v)[NH][4]) {
+// shared sets and the densities from the level's contiguous copy (NS <= 16);
+// otherwise both from each slot's record.
+// tab is uniform and i the lane's wavenumber, so that a row's address is a
+// scalar base plus the lane's 32-bit offset: no address arithmetic in the
+// vector unit.
+template <int NS>
+__device__ __forceinline__ void loadRows(const double* __restrict__ tab, unsigned i,
+                                         const LevelSpecies* __restrict__ d, double (&v)[NS][4]) {
 #pragma unroll
-  for (int s = 0; s < NH; ++s)
+  for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[s][q] = tab[size_t(d[s].block[q]) << 6];
+    for (int q = 0; q < 4; ++q) v[s][q] = (tab + (size_t(d[s].block[q]) << 6))[i];
 }
 
-template <int NH>
-__device__ __forceinline__ double kappaFrom(const double (&v)[NH][4], const LevelSpecies* __restrict__ d,
-                                            const LevelState& lev, StencilGroups groups);
-
-template <int NH>
-__device__ __forceinline__ double kappaTerms(const double* __restrict__ tab, size_t stride,
-                                             const LevelSpecies* __restrict__ d, const LevelState& lev,
-                                             StencilGroups groups, bool reload, double (&v)[NH][4]) {
-  if (reload) loadRows<NH>(tab, d, v);
-  return kappaFrom<NH>(v, d, lev, groups);
+// Slot s's weights out of the two groups' sets.  The model lists the smaller
+// group's species last, so the first NS - NS / 2 slots are always the first
+// group's.  The choice is uniform: made on the words' bits it stays in the
+// scalar unit (on values the compiler may make it per lane).
+template <int NS>
+__device__ __forceinline__ double groupWeight(const double (&a)[4], const double (&b)[4], StencilGroups groups, int s,
+                                              int q) {
+  if (s < NS - NS / 2) return a[q];
+  const bool one = (groups.group1 >> s) & 1u;
+  const int hi = one ? __double2hiint(b[q]) : __double2hiint(a[q]);
+  const int lo = one ? __double2loint(b[q]) : __double2loint(a[q]);
+  return __hiloint2double(hi, lo);
 }
 
-template <int NH>
-__device__ __forceinline__ double kappaFrom(const double (&v)[NH][4], const LevelSpecies* __restrict__ d,
-                                            const LevelState& lev, StencilGroups groups) {
-  double k = 0.0;
+// x_s for every slot, f(s, x)
+template <int NS, class F>
+__device__ __forceinline__ void slotExponents(const double (&v)[NS][4], const LevelSpecies* __restrict__ d,
+                                              const LevelState& lev, StencilGroups groups, F&& f) {
   if (groups.grouped) {
     double a[4], b[4];
 #pragma unroll
@@ -188,24 +174,28 @@ __device__ __forceinline__ double kappaFrom(const double (&v)[NH][4], const Leve
       b[q] = lev.group_w[1][q];
     }
 #pragma unroll
-    for (int s = 0; s < NH; ++s) {
-      const bool one = (groups.group1 >> s) & 1u;
-      double x = fma(one ? b[0] : a[0], v[s][0], lev.log2_n[s]);
-      x = fma(one ? b[1] : a[1], v[s][1], x);
-      x = fma(one ? b[2] : a[2], v[s][2], x);
-      x = fma(one ? b[3] : a[3], v[s][3], x);
-      k += pow2Opacity(x);
+    for (int s = 0; s < NS; ++s) {
+      double x = lev.log2_n[s];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x = fma(groupWeight<NS>(a, b, groups, s, q), v[s][q], x);
+      f(s, x);
     }
   } else {
 #pragma unroll
-    for (int s = 0; s < NH; ++s) {
-      double x = fma(d[s].w[0], v[s][0], d[s].log2_n);
-      x = fma(d[s].w[1], v[s][1], x);
-      x = fma(d[s].w[2], v[s][2], x);
-      x = fma(d[s].w[3], v[s][3], x);
-      k += pow2Opacity(x);
+    for (int s = 0; s < NS; ++s) {
+      double x = d[s].log2_n;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x = fma(d[s].w[q], v[s][q], x);
+      f(s, x);
     }
   }
+}
+
+template <int NS>
+__device__ __forceinline__ double kappaFrom(const double (&v)[NS][4], const LevelSpecies* __restrict__ d,
+                                            const LevelState& lev, StencilGroups groups) {
+  double k = 0.0;
+  slotExponents<NS>(v, d, lev, groups, [&](int, double x) { k += pow2Opacity(x); });
   return k;
 }
 
@@ -262,13 +252,14 @@ __device__ __forceinline__ double cloudLayer(const Extras& ex, const double (&cf
 // and densities from each slot's record.
 constexpr int kChunk = int(kSlotChunk);
 
-__device__ __forceinline__ double chunkedKappa(const double* __restrict__ tab, size_t stride,
+__device__ __forceinline__ double chunkedKappa(const double* __restrict__ tab, unsigned i,
                                                const LevelSpecies* __restrict__ d, const LevelState& lev,
                                                int nb_chunks) {
   double k = 0.0;
   for (int c = 0; c < nb_chunks; ++c, d += kChunk) {
     double v[kChunk][4];
-    k += kappaTerms<kChunk>(tab, stride, d, lev, StencilGroups{0u, 0u}, true, v);      // per-slot records
+    loadRows<kChunk>(tab, i, d, v);
+    k += kappaFrom<kChunk>(v, d, lev, StencilGroups{0u, 0u});                          // per-slot records
   }
   return k;
 }

@@ -38,36 +38,55 @@ struct Extras {
 // Per level: temperature and altitude of the model atmosphere, and whether
 // any stencil slot's table rows differ from the previous level's (always at
 // level 0): the kernels then reload every slot's rows at once, so one scalar
-// decides and the loads issue together.
-struct LevelState {
-  double temperature;
+// decides and the loads issue together.  What the forward kernels read comes
+// first, in whole lines of the scalar cache.
+struct alignas(64) LevelState {
   double inv_temperature;
+  // half the thickness of the layer below this level; 0 at level 0, and where
+  // neither level holds a tabulated absorber (no opacity: an exact 0)
+  double half_dz;
   double altitude;
   double rayleigh_density;   // number density of the Rayleigh scatterer (transmission)
   uint32_t reload;           // bit s: slot s's rows changed
-  uint32_t pad;
+  uint32_t absorbers;        // slots of non-zero density
+  // a layer's cloud optical depth as this level's term: 1 for emission,
+  // 1 / (z_l - z_{l-1}) for transmission (an extinction, cloud_model.h:67-88)
+  double cloud_scale;
+  double temperature;
+  double pad;
+  // group_w and log2_n below in the steps and with the bias of the LDS
+  // exponential table (exp_table.h): w x 128, tableDensity(log2 n)
+  double table_w[2][4];
+  double table_n[16];
+  // the weights and densities for the reduced-precision tables (LevelSpecies32 values)
+  float group_w32[2][4];
+  float log2_n32[16];
+  // per cloud model its optical-depth weight in the layer below this level
+  // (zero at level 0 and outside the cloud)
+  double cloud_w[kMaxClouds];
   // bilinear weights x log2(10) (as LevelSpecies::w) shared by every slot of
   // stencil group 0 and 1 (StencilGroups): slots whose species share a table
   // grid have identical weights at every level
   double group_w[2][4];
   // LevelSpecies::log2_n of slots 0-15, contiguous: one scalar load per level
   double log2_n[16];
-  // the same two for the reduced-precision tables (LevelSpecies32 values)
-  float group_w32[2][4];
-  float log2_n32[16];
   // LevelSpeciesAdjoint::u shared by the slots of stencil group 0 and 1
   double group_u[2][4];
   // the H- continuum's weights of its seven per-wavenumber rows: the H-
   // density, then 1e-29 (5040/T)^((i+1)/2) p_e n_H for i = 1..6 (all zero
   // where the level holds no H-)
   double hminus_c[7];
-  // clouds: per cloud model its optical-depth weight in the layer below this
-  // level (zero at level 0 and outside the cloud), and the factor that turns
-  // that layer's cloud optical depth into this level's term: 1 for emission,
-  // 1 / (z_l - z_{l-1}) for transmission (an extinction, cloud_model.h:67-88)
-  double cloud_w[kMaxClouds];
-  double cloud_scale;
 };
+
+// log2 n in the steps and with the bias of the LDS exponential table, kept to
+// where no slot's exponent leaves the table's range, whatever the
+// cross-section (between 1e-200, the tables' floor, and FP32's largest
+// value).  A density below 2^-340, or of zero, counts as 2^-340: some 1e-122
+// of opacity, far below the last bit of any other term.
+constexpr double kTableSteps = 128.0, kTableBias = 1024.0 * kTableSteps;
+constexpr double tableDensity(double log2_n) {
+  return (log2_n < -340.0 ? -340.0 : log2_n > 850.0 ? 850.0 : log2_n) * kTableSteps + kTableBias;
+}
 
 // log2 of a zero effective density in the FP64 stencil records: finite, so
 // that the kernels' exponentials need no clamp, and low enough that
@@ -168,14 +187,14 @@ constexpr size_t stencilSlots(size_t species) {
   return species == 0 ? 1 : species <= kMaxSlots ? species : (species + kSlotChunk - 1) / kSlotChunk * kSlotChunk;
 }
 
-// f(std::integral_constant<int, NS>) for the slot count ns in 1 .. kMaxSlots;
+// f(std::integral_constant<int, NS>) for the slot count ns in NS .. Last;
 // false when it is none of them
-template <int NS = 1, class F>
+template <int NS = 1, int Last = int(kMaxSlots), class F>
 bool withSlots(size_t ns, F&& f) {
-  if constexpr (NS > int(kMaxSlots)) {
+  if constexpr (NS > Last) {
     return false;
   } else {
-    if (ns != size_t(NS)) return withSlots<NS + 1>(ns, f);
+    if (ns != size_t(NS)) return withSlots<NS + 1, Last>(ns, f);
     f(std::integral_constant<int, NS>{});
     return true;
   }
@@ -200,7 +219,8 @@ struct BatchModel {
   double bottom_radius;          // transmission: R_p (cm)
   double star_radius;            // transmission: R_* (cm)
   double inflation;              // added variance (error inflation), or 0
-  double pad[2];
+  double min_inv_temperature;    // 1 / T of the hottest level
+  double pad;
   CloudSpec clouds;              // the point's cloud models (their weights per level are in its LevelState)
 };
 
@@ -236,8 +256,9 @@ struct StagePlan {
 struct BatchLaunch {
   int block = 256;               // threads per workgroup
   int tile = 256;                // wavenumbers per work item
-  int grid = 0;                  // persistent workgroups
+  int grid = 0;                  // workgroups (transmission: persistent)
   int group = 32;                // points per group of the work-item order (transmission)
+  int split = 1;                 // emission: wavefronts that share one tile's levels
 };
 
 // Per bin of every observation, in observation order: the folded operator
@@ -427,6 +448,7 @@ class DeviceEngine {
   bool use_scratch_ = false;
   unsigned char* scratch_ = nullptr;             // this device's static scratch array
   void upload();                                 // staging -> device, on the stream
+  double hottestLevel() const;                   // smallest 1 / T of the staged levels
   void beginTimed();
   void endTimed();
   void launchBins(int mode, double star_temperature, double depth_scale, double inflation, double* const* bins_dev);
@@ -490,7 +512,8 @@ class DeviceEngine {
   // (transmission with keep: also each kept tile's reach, int32
   // [point][tiles of 64][paths], the largest last segment of every path)
   void launchBatchSpectrum(ModelKind kind, size_t batch, const BatchLaunch& launch, size_t first = 0,
-                           float* keep = nullptr, size_t nu_first = 0, size_t nu_count = 0, int* reach = nullptr);
+                           float* keep = nullptr, size_t nu_first = 0, size_t nu_count = 0, int* reach = nullptr,
+                           bool adjoint = false);
   void launchBatchRest(ModelKind kind, size_t batch, size_t first = 0);
   BatchLaunch tuned(ModelKind kind, size_t batch);
   BatchLaunch tune(ModelKind kind, size_t batch);

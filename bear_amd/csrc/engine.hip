@@ -14,12 +14,14 @@
 // chord lengths) that is copied in one transfer.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
 
 #include "device_math.h"
+#include "emission_sweep.h"
 #include "engine.h"
 
 namespace bear_amd {
@@ -42,11 +44,11 @@ void check(hipError_t e, const char* what) {
   raise(code, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Single-point emission: one wavefront per workgroup.  The grid holds more
-// wavefronts than the chip's slots at the kernel's occupancy (4 per SIMD at
-// 103 VGPRs), and single-wavefront workgroups let the dispatcher refill each
-// freed slot at once (4 % faster than 256 at 400,000 wavenumbers).
-constexpr int kBlock = 64;
+// Single-point emission: workgroups of two wavefronts, the smallest whose
+// exponential tables (16 KiB each) leave LDS for 16 wavefronts per CU
+constexpr int kBlock = 128;
+// Few tiles: workgroups of 4 or 8 wavefronts share one tile's levels
+constexpr int kSplitBlock = 512;
 // Single-point transmission: workgroups of 8 wavefronts share one tile's
 // segment extinction sums in LDS (S[segment][tile], rows padded to
 // chordSegments) and the partial effective heights [kTransmissionBlock /
@@ -56,8 +58,7 @@ size_t transmissionLds(size_t nb_levels, size_t tile) {
   return (size_t(chordSegments(int(nb_levels))) + kTransmissionBlock / tile) * tile * sizeof(double);
 }
 
-// Emission spectrum epilogue: the flux F = 2 pi (mu1 w1 I1 + mu2 w2 I2) 1e-3 s
-// (short_characteristics.cpp:117-122) is kept for the bins; the optional
+// Emission spectrum epilogue: the flux is kept for the bins; the optional
 // high-resolution output is F per micron (radiative_transfer.h:58-60) for
 // emission (mode 0) or the eclipse depth F / F_star (Rp/Rs)^2 1e6
 // (secondary_eclipse.cpp:249-251, mode 1).
@@ -70,10 +71,8 @@ struct SpectrumOut {
   const double* star;
 };
 
-__device__ __forceinline__ void writeFlux(int i, double nu, double i1, double i2, double scaling,
-                                          const double* wavelength, const SpectrumOut& out, double* flux,
-                                          double* spectrum) {
-  const double f = 2.0 * kPi * (i1 * kMu1 * kW + i2 * kMu2 * kW) * 1e-3 * scaling;
+__device__ __forceinline__ void writeFlux(int i, double nu, double f, const double* wavelength,
+                                          const SpectrumOut& out, double* flux, double* spectrum) {
   flux[i] = f;
   if (spectrum) {
     if (out.mode == 1) {
@@ -87,91 +86,76 @@ __device__ __forceinline__ void writeFlux(int i, double nu, double i1, double i2
   }
 }
 
-// Fused opacity + emission radiative transfer, one wavenumber per thread,
-// levels bottom to top (short_characteristics.cpp:39-125).  The four table
-// values of every stencil slot stay in registers from level to level and are
-// reloaded only where the rows change, so each table row is read about once
-// per thread; kappa and the intensities never leave registers.  The next
-// level's rows are requested as soon as this level's kappa is formed, so
-// that their latency passes under this layer's Planck function and
-// attenuation factors.  The stencil fields are wave-uniform (scalar loads).  EX: the extras (H- continuum,
-// clouds) are formed once per thread and added per level and layer: the H-
-// term to kappa, the cloud optical depth to the layer's
-// (short_characteristics.cpp:75-76).
-template <int NS, bool EX>
-__global__ __launch_bounds__(kBlock) void emissionKernelCached(
+// Fused opacity + emission radiative transfer (emission_sweep.h), one
+// wavenumber per lane.  The four table values of every stencil slot stay in
+// registers from level to level and are reloaded only where the rows change,
+// so each table row is read about once per thread; kappa and the transfer
+// never leave registers.  The stencil fields are wave-uniform (scalar loads).
+// EX: the extras (H- continuum, clouds) are formed once per thread and added
+// per level and layer: the H- term to kappa, the cloud optical depth to the
+// layer's (short_characteristics.cpp:75-76).  kSplit: a workgroup is one tile
+// of 64 wavenumbers with the levels split over its wavefronts.
+template <class Op, bool EX, bool kSplit>
+__device__ __forceinline__ void emissionPoint(Op& op, const double* __restrict__ wavenumber,
+                                              const double* __restrict__ wavelength, const Extras& ex,
+                                              const LevelState* __restrict__ levels,
+                                              const LevelSpecies* __restrict__ species, StencilGroups groups,
+                                              int nb_levels, int n, double min_inv_t, double scaling,
+                                              const SpectrumOut& out, double* __restrict__ flux,
+                                              double* __restrict__ spectrum, int i, bool valid, double* part,
+                                              const double* copy) {
+  const double nu = wavenumber[i];
+  const Column col = columnAt(copy, nu, min_inv_t);
+  double hm[7], cf[kMaxClouds];
+  if (EX) loadExtras(ex, i, n, wavelength[i], hm, cf);
+  LayerRun run;
+  double b_top;
+  if constexpr (kSplit) {
+    run = sweepSplit<Op, EX>(op, species, levels, groups, nb_levels, col, ex, hm, cf, i, n, part, b_top);
+    valid = valid && threadIdx.x < 64;
+  } else {
+    run = sweepColumn<Op, EX>(op, species, levels, groups, nb_levels, col, ex, hm, cf, i, n, b_top);
+  }
+  if (valid)
+    writeFlux(i, nu, columnFlux(b_top + run.s1, b_top + run.s2, scaling), wavelength, out, flux, spectrum);
+}
+
+template <int NS, bool EX, bool kSplit>
+__global__ __launch_bounds__((kSplit ? kSplitBlock : kBlock), (sweepWaves<Opacity64<NS>, EX>())) void emissionKernelCached(
     const double* __restrict__ wavenumber, const double* __restrict__ wavelength,
     const double* __restrict__ tables, size_t stride, Extras ex,
     const LevelState* __restrict__ levels, const LevelSpecies* __restrict__ species, StencilGroups groups,
-    int nb_levels, int n, double scaling, SpectrumOut out, double* __restrict__ flux, double* __restrict__ spectrum) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const double nu = wavenumber[i];
-  const double* tab = tables + i;
-  const double b_num = kPlanckC1 * nu * nu * nu;
-  const double x_nu = -(6.62606896e-27 * nu * 2.99792458e10 / 1.3806504e-16) * kLog2E;
-  double v[NS][4];
-  double hm[7], cf[kMaxClouds];
-  if (EX) loadExtras(ex, i, n, wavelength[i], hm, cf);
-  loadRows<NS>(tab, species, v);
-  double k_prev = kappaFrom<NS>(v, species, levels[0], groups);
-  if (EX && ex.hminus) k_prev += hminusKappa(hm, levels[0]);
-  if (nb_levels > 1 && levels[1].reload) loadRows<NS>(tab, species + NS, v);
-  double b_prev = planckAt(b_num, x_nu, levels[0].inv_temperature);
-  double z_prev = levels[0].altitude;
-  double i1 = b_prev, i2 = b_prev;
-  for (int l = 1; l < nb_levels; ++l) {
-    const LevelSpecies* d = species + size_t(l) * NS;
-    double k_next = kappaFrom<NS>(v, d, levels[l], groups);
-    if (EX && ex.hminus) k_next += hminusKappa(hm, levels[l]);
-    if (l + 1 < nb_levels && levels[l + 1].reload) loadRows<NS>(tab, d + NS, v);
-    const double b_next = planckAt(b_num, x_nu, levels[l].inv_temperature);
-    const double z_next = levels[l].altitude;
-    double tau = (z_next - z_prev) * (k_next + k_prev) * 0.5;
-    if (EX) tau += cloudLayer(ex, cf, levels[l], l, i, n);
-    shortCharacteristicsLayer(tau, b_prev, b_next, i1, i2);
-    k_prev = k_next;
-    b_prev = b_next;
-    z_prev = z_next;
-  }
-  writeFlux(i, nu, i1, i2, scaling, wavelength, out, flux, spectrum);
+    int nb_levels, int n, double min_inv_t, double scaling, SpectrumOut out, double* __restrict__ flux,
+    double* __restrict__ spectrum) {
+  extern __shared__ double part[];
+  __shared__ double exp_table[kExpTable];
+  fillExpTable(exp_table);
+  const int at = kSplit ? blockIdx.x * 64 + (threadIdx.x & 63) : blockIdx.x * kBlock + threadIdx.x;
+  const int i = min(at, n - 1);                          // idle lanes follow the last column
+  Opacity64<NS> op;
+  op.init(tables, nullptr, stride, i, expCopy(exp_table));
+  emissionPoint<Opacity64<NS>, EX, kSplit>(op, wavenumber, wavelength, ex, levels, species, groups, nb_levels, n,
+                                           min_inv_t, scaling, out, flux, spectrum, i, at < n, part,
+                                           expCopy(exp_table));
 }
 
 // The same for any number of species, without the register cache.
-__global__ __launch_bounds__(kBlock) void emissionKernel(
+template <bool kSplit>
+__global__ __launch_bounds__(kSplit ? kSplitBlock : kBlock) void emissionKernel(
     const double* __restrict__ wavenumber, const double* __restrict__ wavelength,
     const double* __restrict__ tables, size_t stride, Extras ex,
     const LevelState* __restrict__ levels, const LevelSpecies* __restrict__ species,
-    int nb_levels, int nb_chunks, int n, double scaling, SpectrumOut out,
+    int nb_levels, int nb_chunks, int n, double min_inv_t, double scaling, SpectrumOut out,
     double* __restrict__ flux, double* __restrict__ spectrum) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const double nu = wavenumber[i];
-  const double* tab = tables + i;
-  const double b_num = kPlanckC1 * nu * nu * nu;
-  const double x_nu = -(6.62606896e-27 * nu * 2.99792458e10 / 1.3806504e-16) * kLog2E;
-  const int stride_species = nb_chunks * kChunk;
-  const bool clouds = ex.clouds.count > 0 || ex.cloud_tau;
-  double hm[7], cf[kMaxClouds];
-  loadExtras(ex, i, n, wavelength[i], hm, cf);
-  double k_prev = chunkedKappa(tab, stride, species, levels[0], nb_chunks);
-  if (ex.hminus) k_prev += hminusKappa(hm, levels[0]);
-  double b_prev = planckAt(b_num, x_nu, levels[0].inv_temperature);
-  double z_prev = levels[0].altitude;
-  double i1 = b_prev, i2 = b_prev;
-  for (int l = 1; l < nb_levels; ++l) {
-    double k_next = chunkedKappa(tab, stride, species + size_t(l) * stride_species, levels[l], nb_chunks);
-    if (ex.hminus) k_next += hminusKappa(hm, levels[l]);
-    const double b_next = planckAt(b_num, x_nu, levels[l].inv_temperature);
-    const double z_next = levels[l].altitude;
-    double tau = (z_next - z_prev) * (k_next + k_prev) * 0.5;
-    if (clouds) tau += cloudLayer(ex, cf, levels[l], l, i, n);
-    shortCharacteristicsLayer(tau, b_prev, b_next, i1, i2);
-    k_prev = k_next;
-    b_prev = b_next;
-    z_prev = z_next;
-  }
-  writeFlux(i, nu, i1, i2, scaling, wavelength, out, flux, spectrum);
+  extern __shared__ double part[];
+  __shared__ double exp_table[kExpTable];
+  fillExpTable(exp_table);
+  const int at = kSplit ? blockIdx.x * 64 + (threadIdx.x & 63) : blockIdx.x * kBlock + threadIdx.x;
+  const int i = min(at, n - 1);
+  OpacityChunked op{tables, unsigned(i), nb_chunks};
+  emissionPoint<OpacityChunked, true, kSplit>(op, wavenumber, wavelength, ex, levels, species, StencilGroups{0u, 0u},
+                                              nb_levels, n, min_inv_t, scaling, out, flux, spectrum, i, at < n, part,
+                                           expCopy(exp_table));
 }
 
 // Transmission: transit depth per wavenumber (transmission_spectrum.cpp:32-154).
@@ -198,8 +182,14 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
     const double* __restrict__ wavelength, Extras ex,
     const LevelState* __restrict__ levels, const LevelSpecies* __restrict__ species, StencilGroups stencil_groups,
     const double* __restrict__ chord, int nb_levels, int n, int tile, double bottom_radius, double star_radius,
-    double* __restrict__ depth, double* __restrict__ spectrum) {
+    double* __restrict__ depth, double* __restrict__ spectrum, int exp_offset) {
   extern __shared__ double lds[];
+  // the exponential table where the levels leave room for it
+  const double* exp_copy = nullptr;
+  if (exp_offset > 0) {
+    fillExpTable(lds + exp_offset);
+    exp_copy = expCopy(lds + exp_offset);
+  }
   const int L = nb_levels;
   const int segments = chordSegments(L), tangents = chordTangents(L);
   double* S = lds;
@@ -213,15 +203,15 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
   const int l1 = min(L, l0 + chunk);
   double last = 0.0;
   if (i < n) {
-    const double* tab = tables + i;
+    Opacity64<NS, false> op;
+    op.init(tables, nullptr, stride, i, exp_copy);
     const double sigma_r = rayleigh ? rayleigh[i] : 0.0;
-    double v[NS][4];
     double hm[7], cf[kMaxClouds];
     if (EX) loadExtras(ex, i, n, wavelength[i], hm, cf);
     for (int l = l0; l < l1; ++l) {
-      double k = kappaTerms<NS>(tab, stride, species + size_t(l) * NS, levels[l], stencil_groups,
-                                l == l0 || levels[l].reload != 0, v) +
-                 sigma_r * levels[l].rayleigh_density;
+      const LevelSpecies* d = species + size_t(l) * NS;
+      if (l == l0 || levels[l].reload != 0) op.load(d);
+      double k = op.form(d, levels[l], stencil_groups) + sigma_r * levels[l].rayleigh_density;
       if (EX) {
         if (ex.hminus) k += hminusKappa(hm, levels[l]);
         if (l > 0) k += cloudLayer(ex, cf, levels[l], l, i, n) * levels[l].cloud_scale;
@@ -713,24 +703,48 @@ void DeviceEngine::launchBins(int mode, double star_temperature, double depth_sc
 namespace {
 bool hasExtras(const Extras& ex) { return ex.hminus || ex.cloud_tau || ex.clouds.count > 0; }
 
-void launchEmission(hipStream_t s, size_t species_stride, int blocks, const double* nu, const double* lam,
+// Wavefronts that share one tile's levels: 8 up to 8 tiles per CU, 4 up to 16
+// per CU (4,096 tiles, 262,144 wavenumbers), so that a launch has 8 to 64
+// wavefronts per CU, else 1.  Beyond, whole columns are the faster.
+int levelSplit(int tiles, int cus) { return tiles <= cus * 8 ? 8 : tiles <= cus * 16 ? 4 : 1; }
+
+void launchEmission(hipStream_t s, size_t species_stride, int cus, const double* nu, const double* lam,
                     const double* tables, size_t stride, const Extras& ex, const LevelState* lev,
-                    const LevelSpecies* spc, StencilGroups groups, int L, int n, double scaling, SpectrumOut out,
-                    double* flux, double* spectrum) {
+                    const LevelSpecies* spc, StencilGroups groups, int L, int n, double min_inv_t, double scaling,
+                    SpectrumOut out, double* flux, double* spectrum) {
+  const int tiles = (n + 63) / 64, split = levelSplit(tiles, cus);
+  const dim3 grid{unsigned(split > 1 ? tiles : (n + kBlock - 1) / kBlock)},
+      block{unsigned(split > 1 ? 64 * split : kBlock)};
+  const size_t lds = split > 1 ? splitPart(split) * sizeof(double) : 0;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, nu, lam, tables, stride, ex, lev, spc, groups, L, n, min_inv_t,
+                       scaling, out, flux, spectrum);
+  };
   const bool cached = withSlots(species_stride, [&](auto ns) {
     constexpr int NS = ns;
-    if (hasExtras(ex))
-      hipLaunchKernelGGL((emissionKernelCached<NS, true>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride,
-                         ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);
-    else
-      hipLaunchKernelGGL((emissionKernelCached<NS, false>), dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride,
-                         ex, lev, spc, groups, L, n, scaling, out, flux, spectrum);
+    if (hasExtras(ex)) {
+      if (split > 1) launch(emissionKernelCached<NS, true, true>);
+      else launch(emissionKernelCached<NS, true, false>);
+    } else {
+      if (split > 1) launch(emissionKernelCached<NS, false, true>);
+      else launch(emissionKernelCached<NS, false, false>);
+    }
   });
-  if (!cached)
-    hipLaunchKernelGGL(emissionKernel, dim3(blocks), dim3(kBlock), 0, s, nu, lam, tables, stride, ex, lev, spc, L,
-                       int(species_stride / kChunk), n, scaling, out, flux, spectrum);
+  if (cached) return;
+  auto any = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, nu, lam, tables, stride, ex, lev, spc, L,
+                       int(species_stride / kChunk), n, min_inv_t, scaling, out, flux, spectrum);
+  };
+  if (split > 1) any(emissionKernel<true>);
+  else any(emissionKernel<false>);
 }
 }  // namespace
+
+double DeviceEngine::hottestLevel() const {
+  double t = levels_host_[0].inv_temperature;
+  for (size_t l = 1; l < nb_levels_; ++l) t = std::min(t, levels_host_[l].inv_temperature);
+  return t;
+}
 
 void DeviceEngine::evaluateEmission(double scaling, double inflation, double* spectrum_dev, double* const* bins_dev) {
   if (transmission_) raise(kInvalidInput, "the engine is configured for transmission");
@@ -742,8 +756,8 @@ void DeviceEngine::evaluateEmission(double scaling, double inflation, double* sp
   const LevelSpecies* spc = reinterpret_cast<const LevelSpecies*>(buf.staging + off_species_);
   const int n = int(n_points_);
   beginTimed();
-  launchEmission(s, species_stride_, (n + kBlock - 1) / kBlock, wavenumber_, wavelength_, tables_, stride_, extras(),
-                 lev, spc, groups_, int(nb_levels_), n, scaling, SpectrumOut{0, 0.0, 0.0, nullptr}, buf.flux, spectrum_dev);
+  launchEmission(s, species_stride_, nb_cus_, wavenumber_, wavelength_, tables_, stride_, extras(), lev, spc, groups_,
+                 int(nb_levels_), n, hottestLevel(), scaling, SpectrumOut{0, 0.0, 0.0, nullptr}, buf.flux, spectrum_dev);
   check(hipGetLastError(), "emission kernel");
   endTimed();
   launchBins(0, 0.0, 0.0, inflation, bins_dev);
@@ -761,8 +775,8 @@ void DeviceEngine::evaluateEclipse(double star_temperature, double radius_ratio,
   const int n = int(n_points_);
   const double depth_scale = radius_ratio * radius_ratio * 1e6;
   beginTimed();
-  launchEmission(s, species_stride_, (n + kBlock - 1) / kBlock, wavenumber_, wavelength_, tables_, stride_, extras(),
-                 lev, spc, groups_, int(nb_levels_), n, 1.0, SpectrumOut{1, 1.0 / star_temperature, depth_scale, nullptr}, buf.flux, spectrum_dev);
+  launchEmission(s, species_stride_, nb_cus_, wavenumber_, wavelength_, tables_, stride_, extras(), lev, spc, groups_,
+                 int(nb_levels_), n, hottestLevel(), 1.0, SpectrumOut{1, 1.0 / star_temperature, depth_scale, nullptr}, buf.flux, spectrum_dev);
   check(hipGetLastError(), "emission kernel");
   endTimed();
   launchBins(1, star_temperature, depth_scale, inflation, bins_dev);
@@ -780,8 +794,8 @@ void DeviceEngine::evaluateEclipseTabulatedStar(double radius_ratio, double* spe
   const int n = int(n_points_);
   const double depth_scale = radius_ratio * radius_ratio * 1e6;
   beginTimed();
-  launchEmission(s, species_stride_, (n + kBlock - 1) / kBlock, wavenumber_, wavelength_, tables_, stride_, extras(),
-                 lev, spc, groups_, int(nb_levels_), n, 1.0, SpectrumOut{2, 0.0, depth_scale, star_}, buf.flux, spectrum_dev);
+  launchEmission(s, species_stride_, nb_cus_, wavenumber_, wavelength_, tables_, stride_, extras(), lev, spc, groups_,
+                 int(nb_levels_), n, hottestLevel(), 1.0, SpectrumOut{2, 0.0, depth_scale, star_}, buf.flux, spectrum_dev);
   check(hipGetLastError(), "emission kernel");
   endTimed();
 }
@@ -819,7 +833,12 @@ void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius
   // tiles of 128 or 64 wavenumbers, the wider one when its LDS (the segment
   // sums and the partials) fits the workgroup
   const int tile = transmissionLds(L, 128) <= lds_limit_ ? 128 : 64;
-  const size_t lds = transmissionLds(L, tile);
+  size_t lds = transmissionLds(L, tile);
+  int exp_offset = 0;
+  if (lds + kExpTable * sizeof(double) <= lds_limit_) {
+    exp_offset = int(lds / sizeof(double));
+    lds += kExpTable * sizeof(double);
+  }
   const int blocks = (n + tile - 1) / tile;
   const Extras ex = extras();
   beginTimed();
@@ -828,11 +847,11 @@ void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius
     if (hasExtras(ex))
       hipLaunchKernelGGL((transmissionKernel<NS, true>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
                          stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
-                         star_radius, buf.flux, spectrum_dev);
+                         star_radius, buf.flux, spectrum_dev, exp_offset);
     else
       hipLaunchKernelGGL((transmissionKernel<NS, false>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
                          stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
-                         star_radius, buf.flux, spectrum_dev);
+                         star_radius, buf.flux, spectrum_dev, exp_offset);
   });
   if (!launched) raise(kInvalidInput, "unsupported number of species for transmission");
   check(hipGetLastError(), "transmission kernel");

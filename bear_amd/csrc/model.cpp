@@ -45,6 +45,38 @@ TabulatedModel::TabulatedModel(const GlobalSettings& global, const ModelSettings
     nb_rows += uint32_t(sources.back().nb_rows);
     species_.push_back(std::move(s));
   }
+  // stencil groups: the species' table grids, at most two distinct ones, the
+  // group of fewer species listed last (the kernels choose weights per slot
+  // for the last half of the slots alone)
+  StencilGroups groups;
+  groups.grouped = species_.size() <= 32;                             // one bit each
+  std::vector<int> group_of(species_.size(), 0);
+  int rep[2] = {-1, -1};
+  for (size_t s = 0; s < species_.size() && groups.grouped; ++s) {
+    int g = -1;
+    for (int k = 0; k < 2 && g < 0; ++k) {
+      if (rep[k] < 0) { rep[k] = int(s); g = k; }
+      else if (species_[s].sameGrid(species_[size_t(rep[k])])) g = k;
+    }
+    if (g < 0) groups.grouped = 0;
+    else group_of[s] = g;
+  }
+  if (groups.grouped) {
+    const size_t second = size_t(std::count(group_of.begin(), group_of.end(), 1));
+    const int last = second * 2 > species_.size() ? 0 : 1;             // the smaller group
+    std::vector<OpacitySpecies> species;
+    std::vector<TableSource> ordered;
+    for (int pass = 0; pass < 2; ++pass)
+      for (size_t s = 0; s < species_.size(); ++s)
+        if ((group_of[s] == last) == (pass == 1)) {
+          if (pass == 1) groups.group1 |= 1u << species.size();
+          if (group_rep_[pass] < 0) group_rep_[pass] = int(species.size());
+          species.push_back(std::move(species_[s]));
+          ordered.push_back(std::move(sources[s]));
+        }
+    species_ = std::move(species);
+    sources = std::move(ordered);
+  }
   // one species at a time: host memory holds one species' FP64 rows (and,
   // with reduced-precision storage, the device one species' FP64 staging)
   engine_.allocateTables(nb_rows, sources.size());
@@ -59,19 +91,6 @@ TabulatedModel::TabulatedModel(const GlobalSettings& global, const ModelSettings
   engine_.uploadHminus(hminus);
   for (OpacitySpecies& s : species_) s.preparePressures(atmosphere_.pressure);   // fixed pressure grid
   engine_.configure(m.nb_levels, species_.size(), transmission);
-  // stencil groups: the species' table grids, at most two distinct ones
-  StencilGroups groups;
-  groups.grouped = 1;
-  for (size_t s = 0; s < species_.size() && groups.grouped; ++s) {
-    int g = -1;
-    for (int k = 0; k < 2 && g < 0; ++k) {
-      if (group_rep_[k] < 0) { group_rep_[k] = int(s); g = k; }
-      else if (species_[s].sameGrid(species_[size_t(group_rep_[k])])) g = k;
-    }
-    if (g < 0) groups.grouped = 0;
-    else groups.group1 |= uint32_t(g) << s;
-  }
-  if (!groups.grouped) groups.group1 = 0;
   engine_.setStencilGroups(groups);
   nb_chem_ = atmosphere_.nbChemistryParameters();
   nb_temp_ = atmosphere_.nbTemperatureParameters();
@@ -103,7 +122,10 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
     lev[l].altitude = atm.altitude[l];
     lev[l].rayleigh_density = n_r;
     // a layer's cloud optical depth as this level's term (cloud_model.h:67-88)
-    if (l > 0) lev[l].cloud_scale = transmission_ ? 1.0 / (atm.altitude[l] - atm.altitude[l - 1]) : 1.0;
+    if (l > 0) {
+      lev[l].cloud_scale = transmission_ ? 1.0 / (atm.altitude[l] - atm.altitude[l - 1]) : 1.0;
+      lev[l].half_dz = (atm.altitude[l] - atm.altitude[l - 1]) * 0.5;
+    }
     if (hminus_)                                    // H-, H and electron densities
       hminusCoefficients(t, atm.nd(l, hminus_ids_[0]), atm.nd(l, hminus_ids_[1]), atm.nd(l, hminus_ids_[2]),
                          lev[l].hminus_c);
@@ -116,7 +138,10 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       lev[l].group_w[g][1] = (1.0 - ft) * fl * log2_ten;
       lev[l].group_w[g][2] = ft * (1.0 - fu) * log2_ten;
       lev[l].group_w[g][3] = ft * fu * log2_ten;
-      for (int k = 0; k < 4; ++k) lev[l].group_w32[g][k] = float(lev[l].group_w[g][k]);
+      for (int k = 0; k < 4; ++k) {
+        lev[l].group_w32[g][k] = float(lev[l].group_w[g][k]);
+        lev[l].table_w[g][k] = lev[l].group_w[g][k] * kTableSteps;
+      }
       const double du = st.dft * log2_ten;
       lev[l].group_u[g][0] = -(1.0 - fl) * du;
       lev[l].group_u[g][1] = -fl * du;
@@ -131,6 +156,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
         const OpacitySpecies& sp = species_[s];
         n = atm.nd(l, sp.species_id);                                 // opacity_species.cpp:407-412
         for (int q : sp.cia_partners) n *= atm.nd(l, q);
+        if (n != 0) ++lev[l].absorbers;
         if (groups.grouped) {
           // same grid as the group's representative: same bracket, own rows
           st = group_st[(groups.group1 >> s) & 1u];
@@ -164,7 +190,10 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
         d.w[2] = ft * (1.0 - fu) * log2_ten;
         d.w[3] = ft * fu * log2_ten;
         d.log2_n = n > 0 ? std::log2(n) : kZeroDensityLog2;
-        if (s < 16) lev[l].log2_n[s] = d.log2_n;
+        if (s < 16) {
+          lev[l].log2_n[s] = d.log2_n;
+          lev[l].table_n[s] = tableDensity(d.log2_n);
+        }
         for (int k = 0; k < 4; ++k) d.block[k] = block[k];
         d.reload = changed;
         d.pad = 0;
@@ -184,6 +213,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       }
       lev[l].reload |= changed << s;
     }
+    if (l > 0 && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
   }
   size_t k = 0;                                                   // forward_model.cpp:184-204
   for (size_t o = 0; o < observations_.size(); ++o) {
@@ -300,6 +330,7 @@ void TabulatedModel::stageBatch(const double* params, size_t batch, size_t strid
       scalars = BatchModel{};
       neglect[b] = setup(p, atm, scalars);
       scalars.inflation = inflation[b];
+      scalars.min_inv_temperature = 1.0 / *std::max_element(atm.temperature.begin(), atm.temperature.end());
       stageLevels(atm, modifiers(p), engine_.batchLevels(b), wide ? engine_.batchSpecies(b) : nullptr,
                   wide ? engine_.batchSpeciesAdjoint(b) : nullptr, wide ? nullptr : engine_.batchSpecies32(b),
                   engine_.batchShifts(b));

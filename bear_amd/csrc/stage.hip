@@ -225,7 +225,10 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
     ls.inv_temperature = 1.0 / t;
     ls.altitude = z[l];
     ls.rayleigh_density = (P.rayleigh_id >= 0 && slot[P.rayleigh_id] >= 0) ? n[slot[P.rayleigh_id]] : 0.0;
-    if (l > 0) ls.cloud_scale = P.kind == int(ModelKind::transmission) ? 1.0 / (z[l] - z[l - 1]) : 1.0;
+    if (l > 0) {
+      ls.cloud_scale = P.kind == int(ModelKind::transmission) ? 1.0 / (z[l] - z[l - 1]) : 1.0;
+      ls.half_dz = (z[l] - z[l - 1]) * 0.5;
+    }
     DeviceStencil gst[2];
     for (int q = 0; q < 2; ++q) {
       if (P.group_grid[q] < 0) continue;
@@ -236,13 +239,17 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       ls.group_w[q][1] = (1.0 - ft) * fl * kLog2Ten;
       ls.group_w[q][2] = ft * (1.0 - fu) * kLog2Ten;
       ls.group_w[q][3] = ft * fu * kLog2Ten;
-      for (int k = 0; k < 4; ++k) ls.group_w32[q][k] = float(ls.group_w[q][k]);
+      for (int k = 0; k < 4; ++k) {
+        ls.group_w32[q][k] = float(ls.group_w[q][k]);
+        ls.table_w[q][k] = ls.group_w[q][k] * kTableSteps;
+      }
       const double du = st.dft * kLog2Ten;
       ls.group_u[q][0] = -(1.0 - fl) * du;
       ls.group_u[q][1] = -fl * du;
       ls.group_u[q][2] = (1.0 - fu) * du;
       ls.group_u[q][3] = fu * du;
     }
+    uint32_t absorbers = 0;
     for (int s = 0; s < P.NS; ++s) {
       double dens = 0.0;
       DeviceStencil st{{0, 0}, {0, 0, 0, 0}, 0.0, 0.0, 0.0, 0.0};
@@ -252,6 +259,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
         dens = slot[sp.species_id] >= 0 ? n[slot[sp.species_id]] : 0.0;       // opacity_species.cpp:407-412
         if (sp.partner0 >= 0) dens *= slot[sp.partner0] >= 0 ? n[slot[sp.partner0]] : 0.0;
         if (sp.partner1 >= 0) dens *= slot[sp.partner1] >= 0 ? n[slot[sp.partner1]] : 0.0;
+        if (dens != 0) ++absorbers;
         st = P.grouped ? gst[(P.group1 >> s) & 1u] : bracket(P, blob, sp.grid, l, t);
         for (int k = 0; k < 4; ++k) row[k] = rowId(P, blob, sp, st.t_pos[k / 2], st.p_pos[k]);
       }
@@ -265,7 +273,10 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
         d.w[2] = ft * (1.0 - fu) * kLog2Ten;
         d.w[3] = ft * fu * kLog2Ten;
         d.log2_n = dens > 0 ? log2(dens) : kZeroDensityLog2;
-        if (s < 16) ls.log2_n[s] = d.log2_n;
+        if (s < 16) {
+          ls.log2_n[s] = d.log2_n;
+          ls.table_n[s] = tableDensity(d.log2_n);
+        }
         for (int k = 0; k < 4; ++k) d.block[k] = block[k];
         d.reload = 0;
         d.pad = 0;
@@ -289,6 +300,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
         d.pad[0] = d.pad[1] = 0;
       }
     }
+    ls.absorbers = absorbers;
   }
   __syncthreads();
 
@@ -312,6 +324,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       bits |= changed << s;
     }
     lev[l].reload = bits;
+    if (l > 0 && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
   }
 
   // the point's scalars and observation shifts (emission.cpp:108-120,
@@ -331,6 +344,9 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       bm.bottom_radius = p[1];
       bm.star_radius = p[2];
     }
+    double hottest = T[0];
+    for (int l = 1; l < L; ++l) hottest = fmax(hottest, T[l]);
+    bm.min_inv_temperature = 1.0 / hottest;
     bm.inflation = P.error_inflation ? pow(10.0, p[P.nb_params - 1]) : 0.0;
     double* shifts = reinterpret_cast<double*>(rec + rec_shifts);
     const int* om = at<int>(blob, P.obs_mods);
