@@ -164,9 +164,9 @@ size_t align(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 }  // namespace
 
-size_t transmissionBatchLds(int L, int tile, bool wide) {
+size_t transmissionBatchLds(int L, int tile, bool wide, int threads) {
   const size_t k = size_t(chordSegments(L)) * tile * (wide ? 8 : 4);
-  return align(k, 8) + size_t(kTransmissionBlock / tile) * tile * sizeof(double);
+  return align(k, 8) + size_t(threads / tile) * tile * sizeof(double);
 }
 
 // ---------------------------------------------------------------- precision
@@ -322,6 +322,7 @@ void DeviceEngine::launchBatchSpectrum(ModelKind kind, size_t batch, const Batch
   a.stride = stride_;
   a.ex = Extras{hminus_, nullptr, CloudSpec{}};          // the clouds' parameters come with each point's record
   a.extras = hminus_ != nullptr || cloud_models_ > 0;
+  a.isothermal = isothermal_;
   a.rec = rec;
   a.chord = batch_chord_;
   a.chord32 = batch_chord32_;
@@ -381,8 +382,8 @@ void DeviceEngine::launchBatchRest(ModelKind kind, size_t batch, size_t first) {
 //     leaves the chip under four rounds of wavefronts, also tiles of 64
 //     wavenumbers with their levels split over 2, 4 or 8 wavefronts
 //   transmission: tile of 64 or 128 wavenumbers within the device's LDS per
-//     workgroup; grid of 1, 2 or 4 workgroups per CU; points taken in groups
-//     of 1 or 4 (each point brings its own chord matrix)
+//     workgroup; FP64: grid of 1, 2 or 4 workgroups per CU; points taken in
+//     groups of 1 or 4 (each point brings its own chord matrix)
 BatchLaunch DeviceEngine::tune(ModelKind kind, size_t batch) {
   hipStream_t s = static_cast<hipStream_t>(stream_);
   const size_t b = std::min<size_t>(batch, 64);
@@ -392,8 +393,10 @@ BatchLaunch DeviceEngine::tune(ModelKind kind, size_t batch) {
     for (int tile : {64, 128}) {
       if (transmissionBatchLds(int(nb_levels_), tile, wide) > lds_limit_) continue;
       for (int group : {1, 4})
-        for (int per_cu : {1, 2, 4})
+        for (int per_cu : {1, 2, 4}) {
+          if (!wide && per_cu > 1) continue;                // one item per workgroup: no grid to choose
           cand.push_back(BatchLaunch{kTransmissionBlock, tile, std::max(8, nb_cus_ * per_cu), group});
+        }
     }
     if (cand.empty()) raise(kInvalidInput, "too many levels for the transmission batch kernel");
   } else {

@@ -95,7 +95,7 @@ __global__ __launch_bounds__((kBatchBlock), (sweepWaves<Op, EX>())) void emissio
     e.clouds = bm->clouds;
     loadExtras(e, i, n, wavelength[i], hm, cf);
   }
-  op.load(species);
+  op.load(species, levels[0], rec.groups);
   double k_prev = op.form(species, levels[0], rec.groups);
   if (EX && e.hminus) k_prev += hminusKappa(hm, levels[0]);
   double b_prev = col.planck(levels[0]), d1 = 0.0, d2 = 0.0;       // I = B at the bottom
@@ -107,7 +107,7 @@ __global__ __launch_bounds__((kBatchBlock), (sweepWaves<Op, EX>())) void emissio
   }
   for (int l = 1; l < nb_levels; ++l) {
     const Species* d = species + size_t(l) * Op::kNS;
-    if (levels[l].reload) op.load(d);
+    if (levels[l].reload) op.load(d, levels[l], rec.groups);
     double k_next = op.form(d, levels[l], rec.groups);
     if (EX && e.hminus) k_next += hminusKappa(hm, levels[l]);
     const double b_next = col.planck(levels[l]);

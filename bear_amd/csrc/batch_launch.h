@@ -29,6 +29,7 @@ struct SpectrumBatch {
   const float* base;
   size_t stride;
   Extras ex;
+  bool isothermal;               // DeviceEngine::setIsothermalStencils
   bool extras;                   // the H- rows or the points' cloud models are in use
   dev::Records rec;
   const double* chord;
@@ -48,6 +49,6 @@ bool launchEmissionSlots9To16(size_t slots, const SpectrumBatch& a);
 bool launchTransmissionSlots1To8(size_t slots, const SpectrumBatch& a);
 bool launchTransmissionSlots9To16(size_t slots, const SpectrumBatch& a);
 
-size_t transmissionBatchLds(int levels, int tile, bool wide);
+size_t transmissionBatchLds(int levels, int tile, bool wide, int threads = kTransmissionBlock);
 
 }  // namespace bear_amd

@@ -136,9 +136,7 @@ __device__ __forceinline__ void starFluxWithDerivative(double nu, double inv_t, 
 // With grouped stencils (StencilGroups) the weights come from the level's two
 // shared sets and the densities from the level's contiguous copy (NS <= 16);
 // otherwise both from each slot's record.
-// tab is uniform and i the lane's wavenumber, so that a row's address is a
-// scalar base plus the lane's 32-bit offset: no address arithmetic in the
-// vector unit.
+// tab is uniform and i the lane's wavenumber.
 template <int NS>
 __device__ __forceinline__ void loadRows(const double* __restrict__ tab, unsigned i,
                                          const LevelSpecies* __restrict__ d, double (&v)[NS][4]) {
@@ -153,13 +151,17 @@ __device__ __forceinline__ void loadRows(const double* __restrict__ tab, unsigne
 // group's.  The choice is uniform: made on the words' bits it stays in the
 // scalar unit (on values the compiler may make it per lane).
 template <int NS>
+__device__ __forceinline__ double groupValue(double a, double b, StencilGroups groups, int s) {
+  if (s < NS - NS / 2) return a;
+  const bool one = (groups.group1 >> s) & 1u;
+  const int hi = one ? __double2hiint(b) : __double2hiint(a);
+  const int lo = one ? __double2loint(b) : __double2loint(a);
+  return __hiloint2double(hi, lo);
+}
+template <int NS>
 __device__ __forceinline__ double groupWeight(const double (&a)[4], const double (&b)[4], StencilGroups groups, int s,
                                               int q) {
-  if (s < NS - NS / 2) return a[q];
-  const bool one = (groups.group1 >> s) & 1u;
-  const int hi = one ? __double2hiint(b[q]) : __double2hiint(a[q]);
-  const int lo = one ? __double2loint(b[q]) : __double2loint(a[q]);
-  return __hiloint2double(hi, lo);
+  return groupValue<NS>(a[q], b[q], groups, s);
 }
 
 // x_s for every slot, f(s, x)

@@ -117,7 +117,7 @@ __device__ __forceinline__ double sweepDown(Op& op, const typename Op::Species* 
     return k;
   };
   int l = runTop(nb_levels, first);
-  op.load(level(l));
+  op.load(level(l), levels[l], groups);
   double k_hi = form(l);
   const double b_top = col.planck(levels[l]);
   double b_hi = b_top;
@@ -125,7 +125,7 @@ __device__ __forceinline__ double sweepDown(Op& op, const typename Op::Species* 
     const int bottom = runTop(nb_levels, r + 1);
     LayerRun run;
     for (; l > bottom; --l) {
-      if (levels[l].reload) op.load(level(l - 1));
+      if (levels[l].reload) op.load(level(l - 1), levels[l - 1], groups);
       const double k_lo = form(l - 1);
       const double b_lo = col.planck(levels[l - 1]);
       double tau = levels[l].half_dz * (k_hi + k_lo);

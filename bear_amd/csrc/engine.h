@@ -58,6 +58,10 @@ struct alignas(64) LevelState {
   // exponential table (exp_table.h): w x 128, tableDensity(log2 n)
   double table_w[2][4];
   double table_n[16];
+  // per stencil group the fractions between its temperature rows and, where
+  // every temperature row has the same pressures, between its pressure rows
+  // (isothermal stencils, Opacity64Isothermal)
+  double fraction_t[2], fraction_p[2];
   // the weights and densities for the reduced-precision tables (LevelSpecies32 values)
   float group_w32[2][4];
   float log2_n32[16];
@@ -319,6 +323,10 @@ class DeviceEngine {
   void configure(size_t nb_levels, size_t nb_species, bool transmission);
   void setStencilGroups(StencilGroups g) { groups_ = g; }
   StencilGroups stencilGroups() const { return groups_; }
+  // every level has the same temperature, and each stencil group's
+  // temperature rows the same pressures: the transmission kernels then keep
+  // two values per slot instead of four
+  void setIsothermalStencils(bool on) { isothermal_ = on && groups_.grouped; }
 
   // pinned staging of the per-evaluation inputs; filled by the caller
   LevelState* levels() { return levels_host_; }
@@ -459,6 +467,7 @@ class DeviceEngine {
   size_t nb_levels_ = 0, nb_species_ = 0, species_stride_ = 0;
   bool transmission_ = false;
   StencilGroups groups_;
+  bool isothermal_ = false;
   double* wavenumber_ = nullptr;
   double* wavelength_ = nullptr;
   double* tables_ = nullptr;

@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
     if (EX) loadExtras(ex, i, n, wavelength[i], hm, cf);
     for (int l = l0; l < l1; ++l) {
       const LevelSpecies* d = species + size_t(l) * NS;
-      if (l == l0 || levels[l].reload != 0) op.load(d);
+      if (l == l0 || levels[l].reload != 0) op.load(d, levels[l], stencil_groups);
       double k = op.form(d, levels[l], stencil_groups) + sigma_r * levels[l].rayleigh_density;
       if (EX) {
         if (ex.hminus) k += hminusKappa(hm, levels[l]);

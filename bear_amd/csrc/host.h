@@ -171,6 +171,7 @@ class OpacitySpecies {
   // same temperatures and, per temperature, the same pressures: bracket()
   // then gives the same fractions for every (p, T)
   bool sameGrid(const OpacitySpecies& other) const;
+  bool equalPressures() const;              // every temperature row lists the same pressures
   // preparePressures' picks: per level and temperature row the two pressure
   // rows and the log-pressure fraction
   struct PressurePick { uint16_t lower, upper; double fraction; };

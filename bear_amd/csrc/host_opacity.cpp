@@ -284,6 +284,16 @@ bool OpacitySpecies::sameGrid(const OpacitySpecies& o) const {
   return true;
 }
 
+bool OpacitySpecies::equalPressures() const {
+  const auto& first = by_temperature.front();
+  for (const auto& row : by_temperature) {
+    if (row.size() != first.size()) return false;
+    for (size_t k = 0; k < row.size(); ++k)
+      if (row[k].pressure != first[k].pressure) return false;
+  }
+  return true;
+}
+
 void OpacitySpecies::bracketTemperature(double t, size_t& lo_i, size_t& hi_i) const {
   lo_i = hi_i = 0;
   if (t < by_temperature.front().front().temperature) {

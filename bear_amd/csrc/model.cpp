@@ -92,6 +92,10 @@ TabulatedModel::TabulatedModel(const GlobalSettings& global, const ModelSettings
   for (OpacitySpecies& s : species_) s.preparePressures(atmosphere_.pressure);   // fixed pressure grid
   engine_.configure(m.nb_levels, species_.size(), transmission);
   engine_.setStencilGroups(groups);
+  bool isothermal = atmosphere_.isothermal();
+  for (int r : group_rep_)
+    if (r >= 0) isothermal = isothermal && species_[size_t(r)].equalPressures();
+  engine_.setIsothermalStencils(isothermal);
   nb_chem_ = atmosphere_.nbChemistryParameters();
   nb_temp_ = atmosphere_.nbTemperatureParameters();
   // cloud modules (emission_init.cpp:72-89); their parameters follow the
@@ -134,6 +138,8 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       const Stencil st = species_[size_t(group_rep_[g])].bracketLevel(l, t);
       group_st[g] = st;
       const double ft = st.f_t, fl = st.f_p_lower, fu = st.f_p_upper;
+      lev[l].fraction_t[g] = ft;
+      lev[l].fraction_p[g] = fl;
       lev[l].group_w[g][0] = (1.0 - ft) * (1.0 - fl) * log2_ten;
       lev[l].group_w[g][1] = (1.0 - ft) * fl * log2_ten;
       lev[l].group_w[g][2] = ft * (1.0 - fu) * log2_ten;

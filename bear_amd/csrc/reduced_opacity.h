@@ -92,7 +92,7 @@ struct Opacity32 {
     if constexpr (Tab::kScaled) return sc[s] * float(*p);
     else return Tab::raw(p);
   }
-  __device__ __forceinline__ void load(const LevelSpecies32* d) {
+  __device__ __forceinline__ void load(const LevelSpecies32* d, const LevelState&, StencilGroups) {
 #pragma unroll
     for (int s = 0; s < NS; ++s)
 #pragma unroll
