@@ -24,6 +24,10 @@
 // overwrites each level's opacity with d logL / d kappa; opacityAdjointKernel
 // then recomputes each level's cross-sections from the tables as the forward
 // kernels do and forms d logL / d n_eff and d logL / dT through the tables.
+// The kernels over kept quantities take one work item per workgroup of one
+// wavefront, levelled by the dispatcher: 32 points of 100 levels, 8 species
+// and 50,000 wavenumbers 5.00 -> 4.46 ms per gradient call against persistent
+// grids of 16 wavefronts per CU.  FP64 issue bounds them (70 to 76 % busy).
 // When one point's kept quantities exceed the budget, emissionAdjointKernel
 // does all of it for each work item, recomputing its forward sweep into a
 // per-workgroup scratch first.
@@ -71,8 +75,7 @@ void deviceFree(void* p) {
 
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
-constexpr int kAdjointWavesPerCu = 16;                 // persistent grids of the table kernels
-constexpr int kRtWavesPerCu = 16;                      // and of the recurrence kernel
+constexpr int kAdjointWavesPerCu = 16;                 // persistent grid of emissionAdjointKernel (its scratch)
 constexpr size_t kPartialBudget = size_t(4) << 30;     // partial sums per chunk when recomputing
 constexpr double kLn2 = 0.693147180559945309417232121458176568075500134;
 constexpr double kInvMu1 = 1.0 / kMu1;
@@ -225,6 +228,42 @@ __device__ __forceinline__ void slotTerms(const LevelSpecies* __restrict__ d, co
       f(s, term(x), y);
     }
   }
+}
+
+// slotTerms for grouped stencils from the rows' pressure steps (loadSteps:
+// the lower row and the step to the upper one, at both temperatures, times
+// log2 10): five operations per slot for the exponent and its slope in the
+// fraction between the temperatures together, where the weighted rows take
+// eight (4.46 -> 4.36 ms for the call above).  t[s] = t_s; returns
+// sum_s t_s y_s.
+template <int NS>
+__device__ __forceinline__ void loadSteps(double (&v)[NS][4]) {
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    v[s][1] = (v[s][1] - v[s][0]) * kLog2Ten;
+    v[s][3] = (v[s][3] - v[s][2]) * kLog2Ten;
+    v[s][0] *= kLog2Ten;
+    v[s][2] *= kLog2Ten;
+  }
+}
+
+template <int NS>
+__device__ __forceinline__ double stepTerms(const LevelState& lev, StencilGroups groups, const double (&v)[NS][4],
+                                            double (&t)[NS]) {
+  constexpr int kFirst = NS - NS / 2;                              // slots that are always group 0's
+  double first = 0.0, rest = 0.0;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double fl = groupValue<NS>(lev.fraction_p[0], lev.fraction_p[1], groups, s);
+    const double fu = groupValue<NS>(lev.fraction_q[0], lev.fraction_q[1], groups, s);
+    const double ft = groupValue<NS>(lev.fraction_t[0], lev.fraction_t[1], groups, s);
+    const double lo = fma(fl, v[s][1], v[s][0]);
+    const double step = fma(fu, v[s][3], v[s][2]) - lo;
+    t[s] = pow2Gradient(fma(ft, step, lo) + lev.log2_n[s]);
+    if (s < kFirst) first = fma(t[s], step, first);
+    else rest = fma(t[s], step * groupValue<NS>(lev.slope_t[0], lev.slope_t[1], groups, s), rest);
+  }
+  return fma(first, lev.slope_t[0], rest);
 }
 
 // Opacity of one level for the backward sweep: kappa = sum_s t_s and
@@ -447,112 +486,109 @@ __global__ __launch_bounds__(kWave) void rtAdjointKernel(const double* __restric
   const int K = kslots;
   const int lane = int(threadIdx.x);
   const size_t level_step = kKeptLevel;
-  const size_t total = nbItems(tiles, batch);
-  for (size_t item = blockIdx.x; item < total; item += gridDim.x) {
-    int m, tile;
-    if (!workItem(item, batch, tiles, m, tile)) continue;          // uniform over the wavefront
-    const int i = tile * kWave + lane;
-    const bool valid = i < n;
-    const int ic = valid ? i : n - 1;                                // idle lanes: zero adjoints, no stores
-    const unsigned char* r = rec.at(m);
-    const BatchModel* bm = reinterpret_cast<const BatchModel*>(r);
-    const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
-    float* kp = keep + keptColumn(m, stride, L, ic);
-    double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
-    const double nu = wavenumber[ic];
-    const double b_num = kPlanckC1 * nu * nu * nu;
-    const double x_nu = -(6.62606896e-27 * nu * 2.99792458e10 / 1.3806504e-16) * kLog2E;
-    const double fb = valid ? fbar[size_t(m) * stride + i] : 0.0;
-    const double unit = 2.0 * kPi * 1e-3;
-    double cf[kMaxClouds], cg[kMaxClouds][3];
+  int m, tile;
+  if (!workItem(blockIdx.x, batch, tiles, m, tile)) return;        // uniform over the wavefront
+  const int i = tile * kWave + lane;
+  const bool valid = i < n;
+  const int ic = valid ? i : n - 1;                                // idle lanes: zero adjoints, no stores
+  const unsigned char* r = rec.at(m);
+  const BatchModel* bm = reinterpret_cast<const BatchModel*>(r);
+  const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
+  float* kp = keep + keptColumn(m, stride, L, ic);
+  double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
+  const double nu = wavenumber[ic];
+  const double b_num = kPlanckC1 * nu * nu * nu;
+  const double x_nu = -(6.62606896e-27 * nu * 2.99792458e10 / 1.3806504e-16) * kLog2E;
+  const double fb = valid ? fbar[size_t(m) * stride + i] : 0.0;
+  const double unit = 2.0 * kPi * 1e-3;
+  double cf[kMaxClouds], cg[kMaxClouds][3];
+  if constexpr (CL) {
+    double hm[7];
+    const Extras e{nullptr, nullptr, bm->clouds};
+    const double lam = wavelength[ic];
+    loadExtras(e, ic, n, lam, hm, cf);
+#pragma unroll
+    for (int c = 0; c < kMaxClouds; ++c) {
+      cg[c][0] = cg[c][1] = cg[c][2] = 0.0;
+      if (c < e.clouds.count && e.clouds.kind[c] == kCloudPowerLaw) {
+        cg[c][0] = cf[c] * (log(lam) - e.clouds.c[c][2]);
+      } else if (c < e.clouds.count && e.clouds.kind[c] == kCloudKH) {
+        const double* k = e.clouds.c[c];
+        const double x = k[2] / lam, xm = pow(x, -k[1]), x2 = pow(x, 0.2);
+        const double fu = cf[c] / (k[0] * xm + x2);
+        cg[c][0] = fu * xm;
+        cg[c][1] = fu * k[0] * xm * log(x);
+        cg[c][2] = fu * (0.2 * x2 - k[1] * k[0] * xm);
+      }
+    }
+  }
+  // kept: d = I - B of both angles and kappa per level, FP32
+  const float* top = kp + size_t(L - 1) * level_step;
+  double b_hi, db_hi;
+  planckAdjoint(b_num, x_nu, levels[L - 1].inv_temperature, b_hi, db_hi);
+  const double s_bar = fb * unit * ((double(top[0]) + b_hi) * (kMu1 * kW) + (double(top[kKeptValue]) + b_hi) * (kMu2 * kW));
+  double ib1 = fb * unit * bm->scaling * (kMu1 * kW);
+  double ib2 = fb * unit * bm->scaling * (kMu2 * kW);
+  double k_hi = top[2 * kKeptValue];
+  double z_hi = levels[L - 1].altitude;
+  double kbar_hi = 0.0, zbar_hi = 0.0, bbar_hi = 0.0;
+  const float* below = kp + size_t(L - 2) * level_step;          // the level below, read one step ahead
+  double d1n = below[0], d2n = below[kKeptValue], kn = below[2 * kKeptValue];
+  for (int l = L - 1; l >= 1; --l) {
+    const double d1p = d1n, d2p = d2n, k_lo = kn;
+    if (l >= 2) {
+      below = kp + size_t(l - 2) * level_step;
+      d1n = below[0];
+      d2n = below[kKeptValue];
+      kn = below[2 * kKeptValue];
+    }
+    double b_lo, db_lo;
+    planckAdjoint(b_num, x_nu, levels[l - 1].inv_temperature, b_lo, db_lo);
+    const double z_lo = levels[l - 1].altitude;
+    const double dz = z_hi - z_lo;
+    const double k_mean = (k_hi + k_lo) * 0.5;
+    double tau = dz * k_mean;
+    if constexpr (CL)
+#pragma unroll
+      for (int c = 0; c < kMaxClouds; ++c) tau = fma(levels[l].cloud_w[c], cf[c], tau);
+    double tbar = 0.0, bbar_lo = 0.0;
+    if (tau != 0) {
+      const double rt = recip(tau);
+      angleAdjoint(tau, rt, kMu1, kInvMu1, d1p, b_lo, b_hi, ib1, tbar, bbar_hi, bbar_lo);
+      angleAdjoint(tau, rt, kMu2, kInvMu2, d2p, b_lo, b_hi, ib2, tbar, bbar_hi, bbar_lo);
+    }
+    const double kbar_lo = tbar * dz * 0.5;
+    kbar_hi += kbar_lo;
+    zbar_hi = fma(tbar, k_mean, zbar_hi);
+    // every contribution to level l is in
+    if (valid) kp[size_t(l) * level_step + 2 * kKeptValue] = float(kbar_hi);
+    double x[4] = {zbar_hi, 0.0, bbar_hi * db_hi, 0.0};
+    emitSums<4>(out + size_t(l) * tiles * K, lane, x, ns + 1, 3);
     if constexpr (CL) {
-      double hm[7];
-      const Extras e{nullptr, nullptr, bm->clouds};
-      const double lam = wavelength[ic];
-      loadExtras(e, ic, n, lam, hm, cf);
+      double xc[4 * kMaxClouds];
 #pragma unroll
       for (int c = 0; c < kMaxClouds; ++c) {
-        cg[c][0] = cg[c][1] = cg[c][2] = 0.0;
-        if (c < e.clouds.count && e.clouds.kind[c] == kCloudPowerLaw) {
-          cg[c][0] = cf[c] * (log(lam) - e.clouds.c[c][2]);
-        } else if (c < e.clouds.count && e.clouds.kind[c] == kCloudKH) {
-          const double* k = e.clouds.c[c];
-          const double x = k[2] / lam, xm = pow(x, -k[1]), x2 = pow(x, 0.2);
-          const double fu = cf[c] / (k[0] * xm + x2);
-          cg[c][0] = fu * xm;
-          cg[c][1] = fu * k[0] * xm * log(x);
-          cg[c][2] = fu * (0.2 * x2 - k[1] * k[0] * xm);
-        }
-      }
-    }
-    // kept: d = I - B of both angles and kappa per level, FP32
-    const float* top = kp + size_t(L - 1) * level_step;
-    double b_hi, db_hi;
-    planckAdjoint(b_num, x_nu, levels[L - 1].inv_temperature, b_hi, db_hi);
-    const double s_bar = fb * unit * ((double(top[0]) + b_hi) * (kMu1 * kW) + (double(top[kKeptValue]) + b_hi) * (kMu2 * kW));
-    double ib1 = fb * unit * bm->scaling * (kMu1 * kW);
-    double ib2 = fb * unit * bm->scaling * (kMu2 * kW);
-    double k_hi = top[2 * kKeptValue];
-    double z_hi = levels[L - 1].altitude;
-    double kbar_hi = 0.0, zbar_hi = 0.0, bbar_hi = 0.0;
-    const float* below = kp + size_t(L - 2) * level_step;          // the level below, read one step ahead
-    double d1n = below[0], d2n = below[kKeptValue], kn = below[2 * kKeptValue];
-    for (int l = L - 1; l >= 1; --l) {
-      const double d1p = d1n, d2p = d2n, k_lo = kn;
-      if (l >= 2) {
-        below = kp + size_t(l - 2) * level_step;
-        d1n = below[0];
-        d2n = below[kKeptValue];
-        kn = below[2 * kKeptValue];
-      }
-      double b_lo, db_lo;
-      planckAdjoint(b_num, x_nu, levels[l - 1].inv_temperature, b_lo, db_lo);
-      const double z_lo = levels[l - 1].altitude;
-      const double dz = z_hi - z_lo;
-      const double k_mean = (k_hi + k_lo) * 0.5;
-      double tau = dz * k_mean;
-      if constexpr (CL)
+        xc[4 * c] = tbar * cf[c];
 #pragma unroll
-        for (int c = 0; c < kMaxClouds; ++c) tau = fma(levels[l].cloud_w[c], cf[c], tau);
-      double tbar = 0.0, bbar_lo = 0.0;
-      if (tau != 0) {
-        const double rt = recip(tau);
-        angleAdjoint(tau, rt, kMu1, kInvMu1, d1p, b_lo, b_hi, ib1, tbar, bbar_hi, bbar_lo);
-        angleAdjoint(tau, rt, kMu2, kInvMu2, d2p, b_lo, b_hi, ib2, tbar, bbar_hi, bbar_lo);
+        for (int k = 0; k < 3; ++k) xc[4 * c + 1 + k] = tbar * cg[c][k];
       }
-      const double kbar_lo = tbar * dz * 0.5;
-      kbar_hi += kbar_lo;
-      zbar_hi = fma(tbar, k_mean, zbar_hi);
-      // every contribution to level l is in
-      if (valid) kp[size_t(l) * level_step + 2 * kKeptValue] = float(kbar_hi);
-      double x[4] = {zbar_hi, 0.0, bbar_hi * db_hi, 0.0};
-      emitSums<4>(out + size_t(l) * tiles * K, lane, x, ns + 1, 3);
-      if constexpr (CL) {
-        double xc[4 * kMaxClouds];
-#pragma unroll
-        for (int c = 0; c < kMaxClouds; ++c) {
-          xc[4 * c] = tbar * cf[c];
-#pragma unroll
-          for (int k = 0; k < 3; ++k) xc[4 * c + 1 + k] = tbar * cg[c][k];
-        }
-        emitSums<4 * kMaxClouds>(out + size_t(l) * tiles * K, lane, xc, cloud_slot0, 4 * kMaxClouds);
-      }
-      k_hi = k_lo;
-      b_hi = b_lo;
-      db_hi = db_lo;
-      z_hi = z_lo;
-      kbar_hi = kbar_lo;
-      zbar_hi = -tbar * k_mean;
-      bbar_hi = bbar_lo;
+      emitSums<4 * kMaxClouds>(out + size_t(l) * tiles * K, lane, xc, cloud_slot0, 4 * kMaxClouds);
     }
-    bbar_hi += ib1 + ib2;                                            // I_0 = B_0
-    if (valid) kp[2 * kKeptValue] = float(kbar_hi);
-    double x[4] = {zbar_hi, s_bar, bbar_hi * db_hi, 0.0};
-    emitSums<4>(out, lane, x, ns + 1, 3);
-    if constexpr (CL) {                                              // no layer below level 0
-      double xc[4 * kMaxClouds] = {};
-      emitSums<4 * kMaxClouds>(out, lane, xc, cloud_slot0, 4 * kMaxClouds);
-    }
+    k_hi = k_lo;
+    b_hi = b_lo;
+    db_hi = db_lo;
+    z_hi = z_lo;
+    kbar_hi = kbar_lo;
+    zbar_hi = -tbar * k_mean;
+    bbar_hi = bbar_lo;
+  }
+  bbar_hi += ib1 + ib2;                                            // I_0 = B_0
+  if (valid) kp[2 * kKeptValue] = float(kbar_hi);
+  double x[4] = {zbar_hi, s_bar, bbar_hi * db_hi, 0.0};
+  emitSums<4>(out, lane, x, ns + 1, 3);
+  if constexpr (CL) {                                              // no layer below level 0
+    double xc[4 * kMaxClouds] = {};
+    emitSums<4 * kMaxClouds>(out, lane, xc, cloud_slot0, 4 * kMaxClouds);
   }
 }
 
@@ -575,51 +611,58 @@ __global__ __launch_bounds__(kWave) void opacityAdjointKernel(const double* __re
   const int K = kslots;                                             // partial row: every level slot
   const int L = nb_levels;
   const int lane = int(threadIdx.x);
-  const size_t total = nbItems(win.count, batch);
-  for (size_t item = blockIdx.x; item < total; item += gridDim.x) {
-    int m, tile;
-    if (!windowItem(item, batch, win, m, tile)) continue;          // uniform over the wavefront
-    const int i = tile * kWave + lane;
-    const bool valid = i < n;
-    const int ic = valid ? i : n - 1;
-    const unsigned char* r = rec.at(m);
-    const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
-    const LevelSpecies* species = reinterpret_cast<const LevelSpecies*>(r + rec.species);
-    const LevelSpeciesAdjoint* extra = reinterpret_cast<const LevelSpeciesAdjoint*>(r + rec.adjoint);
-    const float* kb = keep + keptAt(win, m, stride, L, ic) + 2 * kKeptValue;
-    double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
-    double v[NS][4];
-    double hm[7];
-    if constexpr (HM)
+  int m, tile;
+  if (!windowItem(blockIdx.x, batch, win, m, tile)) return;        // uniform over the wavefront
+  const int i = tile * kWave + lane;
+  const bool valid = i < n;
+  const int ic = valid ? i : n - 1;
+  const unsigned char* r = rec.at(m);
+  const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
+  const LevelSpecies* species = reinterpret_cast<const LevelSpecies*>(r + rec.species);
+  const LevelSpeciesAdjoint* extra = reinterpret_cast<const LevelSpeciesAdjoint*>(r + rec.adjoint);
+  const float* kb = keep + keptAt(win, m, stride, L, ic) + 2 * kKeptValue;
+  double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
+  double v[NS][4];
+  double hm[7];
+  if constexpr (HM)
 #pragma unroll
-      for (int r = 0; r < 7; ++r) hm[r] = hminus[size_t(r) * n + ic];
-    // d logL / d kappa streams from HBM: read two levels ahead
-    double kb1 = kb[0], kb2 = L > 1 ? kb[kKeptLevel] : 0.0;
-    for (int l = 0; l < L; ++l) {
-      const double kbar = valid ? kb1 : 0.0;
-      const LevelSpecies* d = species + size_t(l) * NS;
-      const LevelSpeciesAdjoint* a = extra + size_t(l) * NS;
-      if (l == 0 || levels[l].reload != 0) loadRows<NS>(tables, unsigned(ic), d, v);
-      kb1 = kb2;
-      if (l + 2 < L) kb2 = kb[size_t(l + 2) * kKeptLevel];
-      double x[KX];
-      double dk = 0.0;
-      // the terms to 1.2e-7 (pow2Gradient): they only weight d logL / d kappa
+    for (int r = 0; r < 7; ++r) hm[r] = hminus[size_t(r) * n + ic];
+  // d logL / d kappa streams from HBM: read two levels ahead
+  double kb1 = kb[0], kb2 = L > 1 ? kb[kKeptLevel] : 0.0;
+  for (int l = 0; l < L; ++l) {
+    const double kbar = valid ? kb1 : 0.0;
+    const LevelSpecies* d = species + size_t(l) * NS;
+    const LevelSpeciesAdjoint* a = extra + size_t(l) * NS;
+    if (l == 0 || levels[l].reload != 0) {
+      loadRows<NS>(tables, unsigned(ic), d, v);
+      if (rec.groups.grouped) loadSteps<NS>(v);
+    }
+    kb1 = kb2;
+    if (l + 2 < L) kb2 = kb[size_t(l + 2) * kKeptLevel];
+    double x[KX];
+    double dk = 0.0;
+    // the terms to 1.2e-7 (pow2Gradient): they only weight d logL / d kappa
+    if (rec.groups.grouped) {
+      double t[NS];
+      dk = stepTerms<NS>(levels[l], rec.groups, v, t);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) x[s] = kbar * t[s];
+    } else {
       slotTerms<NS, true>(d, a, levels[l], rec.groups, v, [&](int s, double ts, double ys) {
         x[s] = kbar * ts;
         dk = fma(ts, ys, dk);
       });
-      x[NS] = kbar * dk * kLn2;
+    }
+    x[NS] = kbar * dk * kLn2;
 #pragma unroll
-      for (int s = NS + 1; s < KX; ++s) x[s] = 0.0;
-      emitSums<KX>(out + size_t(l) * tiles * K, lane, x, 0, NS + 1);
-      if constexpr (HM) {
-        double xh[8];
+    for (int s = NS + 1; s < KX; ++s) x[s] = 0.0;
+    emitSums<KX>(out + size_t(l) * tiles * K, lane, x, 0, NS + 1);
+    if constexpr (HM) {
+      double xh[8];
 #pragma unroll
-        for (int r = 0; r < 7; ++r) xh[r] = kbar * hm[r];
-        xh[7] = 0.0;
-        emitSums<8>(out + size_t(l) * tiles * K, lane, xh, NS + 4, 8);
-      }
+      for (int r = 0; r < 7; ++r) xh[r] = kbar * hm[r];
+      xh[7] = 0.0;
+      emitSums<8>(out + size_t(l) * tiles * K, lane, xh, NS + 4, 8);
     }
   }
 }
@@ -656,23 +699,24 @@ __global__ __launch_bounds__(kBlock) void adjointReduceKernel(const double* __re
 // hminus: the H- continuum's rows (kept forward only), its sums in slots
 // NS+4 .. NS+10 of kslots per level
 template <int NS>
-void launchAdjoint(bool kept, dim3 grid, dim3 rt_grid, hipStream_t s, const double* nu, const double* lam,
+void launchAdjoint(bool kept, dim3 grid, hipStream_t s, const double* nu, const double* lam,
                    const double* tables, size_t stride, Records rec, int L, int n, int tiles, int batch,
                    const double* fbar, double* buffer, double* partial, const double* hminus, int kslots,
                    int cloud_slot0) {
   if (kept) {
+    const dim3 items(unsigned(nbItems(tiles, batch)));
     float* kept_values = reinterpret_cast<float*>(buffer);
     if (cloud_slot0 >= 0)
-      hipLaunchKernelGGL(rtAdjointKernel<true>, rt_grid, dim3(kWave), 0, s, nu, rec, L, n, stride, tiles, batch, NS,
+      hipLaunchKernelGGL(rtAdjointKernel<true>, items, dim3(kWave), 0, s, nu, rec, L, n, stride, tiles, batch, NS,
                          kslots, fbar, kept_values, partial, lam, cloud_slot0);
     else
-      hipLaunchKernelGGL(rtAdjointKernel<false>, rt_grid, dim3(kWave), 0, s, nu, rec, L, n, stride, tiles, batch, NS,
+      hipLaunchKernelGGL(rtAdjointKernel<false>, items, dim3(kWave), 0, s, nu, rec, L, n, stride, tiles, batch, NS,
                          kslots, fbar, kept_values, partial, lam, cloud_slot0);
     if (hminus)
-      hipLaunchKernelGGL((opacityAdjointKernel<NS, true>), grid, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
+      hipLaunchKernelGGL((opacityAdjointKernel<NS, true>), items, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
                          wholeGrid(tiles), batch, kept_values, hminus, kslots, partial);
     else
-      hipLaunchKernelGGL(opacityAdjointKernel<NS>, grid, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
+      hipLaunchKernelGGL(opacityAdjointKernel<NS>, items, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
                          wholeGrid(tiles), batch, kept_values, hminus, kslots, partial);
   } else {
     hipLaunchKernelGGL(emissionAdjointKernel<NS>, grid, dim3(kWave), 0, s, nu, tables, stride, rec, L, n, tiles,
@@ -715,34 +759,31 @@ __global__ __launch_bounds__(kWave) void tangentAdjointKernel(Records rec, int n
   const int L = nb_levels, K = kslots;
   const int lane = int(threadIdx.x);
   const size_t level_step = kKeptLevel;
-  const size_t total = nbItems(win.count, batch);
-  for (size_t item = blockIdx.x; item < total; item += gridDim.x) {
-    int m, tile;
-    if (!windowItem(item, batch, win, m, tile)) continue;          // uniform over the wavefront
-    const int i = tile * kWave + lane;
-    const bool valid = i < n;
-    const int ic = valid ? i : n - 1;                                // idle lanes: zero adjoints, no stores
-    const unsigned char* r = rec.at(m);
-    const BatchModel* bm = reinterpret_cast<const BatchModel*>(r);
-    const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
-    float* kp = keep + keptAt(win, m, stride, L, ic);
-    double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
-    const double fb = valid ? fbar[size_t(m) * stride + i] : 0.0;
-    const double e = fb * 1e6 / (bm->star_radius * bm->star_radius);
-    const double r0 = bm->bottom_radius;
-    for (int t = 0; t < L - 1; ++t) {
-      float* kt = kp + size_t(t) * level_step + kKeptValue;
-      const double tr = pow2(-double(*kt) * kLog2E);
-      const double zl = levels[t > 0 ? t - 1 : 0].altitude, zu = levels[t + 1].altitude;
-      const double ct = (r0 + levels[t].altitude) * (zu - zl);
-      if (valid) *kt = float(e * ct * tr);
-      double x4[4] = {e * (1.0 - tr), 0.0, 0.0, 0.0};
-      emitSums<4>(out + size_t(t) * tiles * K, lane, x4, ns + 1, 2);
-    }
-    const double d = valid ? depth[size_t(m) * stride + i] : 0.0;
-    double x4[4] = {e, fb * d, 0.0, 0.0};
-    emitSums<4>(out + size_t(L - 1) * tiles * K, lane, x4, ns + 1, 2);
+  int m, tile;
+  if (!windowItem(blockIdx.x, batch, win, m, tile)) return;        // uniform over the wavefront
+  const int i = tile * kWave + lane;
+  const bool valid = i < n;
+  const int ic = valid ? i : n - 1;                                // idle lanes: zero adjoints, no stores
+  const unsigned char* r = rec.at(m);
+  const BatchModel* bm = reinterpret_cast<const BatchModel*>(r);
+  const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
+  float* kp = keep + keptAt(win, m, stride, L, ic);
+  double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;         // level l: + l * tiles * K
+  const double fb = valid ? fbar[size_t(m) * stride + i] : 0.0;
+  const double e = fb * 1e6 / (bm->star_radius * bm->star_radius);
+  const double r0 = bm->bottom_radius;
+  for (int t = 0; t < L - 1; ++t) {
+    float* kt = kp + size_t(t) * level_step + kKeptValue;
+    const double tr = pow2(-double(*kt) * kLog2E);
+    const double zl = levels[t > 0 ? t - 1 : 0].altitude, zu = levels[t + 1].altitude;
+    const double ct = (r0 + levels[t].altitude) * (zu - zl);
+    if (valid) *kt = float(e * ct * tr);
+    double x4[4] = {e * (1.0 - tr), 0.0, 0.0, 0.0};
+    emitSums<4>(out + size_t(t) * tiles * K, lane, x4, ns + 1, 2);
   }
+  const double d = valid ? depth[size_t(m) * stride + i] : 0.0;
+  double x4[4] = {e, fb * d, 0.0, 0.0};
+  emitSums<4>(out + size_t(L - 1) * tiles * K, lane, x4, ns + 1, 2);
 }
 
 // Step 2: one workgroup of 256 threads per (64 x 64 block of (q, t) with
@@ -890,85 +931,82 @@ __global__ __launch_bounds__(kWave) void segmentAdjointKernel(Records rec, const
   const int rows = segmentRows(L);
   const int lane = int(threadIdx.x);
   const size_t level_step = kKeptLevel;
-  const size_t total = nbItems(win.count, batch);
-  for (size_t item = blockIdx.x; item < total; item += gridDim.x) {
-    int m, tile;
-    if (!windowItem(item, batch, win, m, tile, 1)) continue;   // uniform; tiles of one point together (its chords)
-    const int i = tile * kWave + lane;
-    const bool valid = i < n;
-    const int ic = valid ? i : n - 1;
-    float* kp = keep + keptAt(win, m, stride, L, ic);
-    const double* c = chord_t + size_t(m) * (L - 1) * rows;
-    double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;
-    const double sr = (rayleigh && valid) ? rayleigh[i] : 0.0;
-    const int* rl = reach + (size_t(m) * tiles + tile) * (L - 1);   // per path: the wavefront's largest last_t
-    double s_hi = 0.0;                                               // S-bar of the segment above
-    // kAdjointSegments segments per pass over the paths (one load of
-    // tau-bar_t and last_t for all of them); chord[q][t] = 0 for t > q and
-    // past the last segment.  Per path, tests uniform over the wavefront:
-    // every lane's path ends below the pass (skipped), or reaches past it
-    // (no masks); otherwise the products are masked lane by lane.
-    for (int qb = (L - 2) / kAdjointSegments * kAdjointSegments; qb >= 0; qb -= kAdjointSegments) {
-      double sb[kAdjointSegments];
+  int m, tile;
+  if (!windowItem(blockIdx.x, batch, win, m, tile, 1)) return;   // uniform; tiles of one point together (its chords)
+  const int i = tile * kWave + lane;
+  const bool valid = i < n;
+  const int ic = valid ? i : n - 1;
+  float* kp = keep + keptAt(win, m, stride, L, ic);
+  const double* c = chord_t + size_t(m) * (L - 1) * rows;
+  double* out = partial + (size_t(m) * L * size_t(tiles) + tile) * K;
+  const double sr = (rayleigh && valid) ? rayleigh[i] : 0.0;
+  const int* rl = reach + (size_t(m) * tiles + tile) * (L - 1);   // per path: the wavefront's largest last_t
+  double s_hi = 0.0;                                               // S-bar of the segment above
+  // kAdjointSegments segments per pass over the paths (one load of
+  // tau-bar_t and last_t for all of them); chord[q][t] = 0 for t > q and
+  // past the last segment.  Per path, tests uniform over the wavefront:
+  // every lane's path ends below the pass (skipped), or reaches past it
+  // (no masks); otherwise the products are masked lane by lane.
+  for (int qb = (L - 2) / kAdjointSegments * kAdjointSegments; qb >= 0; qb -= kAdjointSegments) {
+    double sb[kAdjointSegments];
 #pragma unroll
-      for (int u = 0; u < kAdjointSegments; ++u) sb[u] = 0.0;
-      const int t_end = min(qb + kAdjointSegments, L - 1);
-      // this lane's tau-bar and last segment of path t, for the paths that
-      // reach the pass (the next one's are loaded while a path's products
-      // run); the others end below every segment of the pass
-      auto column = [&](int t) { return kp + size_t(t) * level_step; };
-      auto next = [&](int t) {                         // the first path from t on that reaches the pass
-        while (t < t_end && rl[t] < qb) ++t;
-        return t;
-      };
-      int t = next(0);
-      double tb = 0.0;
-      int last = -1;
-      if (t < t_end) {
-        tb = double(column(t)[kKeptValue]);
-        last = int(column(t)[2 * kKeptValue]);
-      }
-      while (t < t_end) {
-        const int t_next = next(t + 1);
-        double tb_next = 0.0;
-        int last_next = -1;
-        if (t_next < t_end) {                          // uniform
-          tb_next = double(column(t_next)[kKeptValue]);
-          last_next = int(column(t_next)[2 * kKeptValue]);
-        }
-        {
-          const double* ct = c + size_t(t) * rows + qb;
-          const int k = last - qb;                     // this lane sums segments qb .. qb + k
-          // Past segment qb + k only the high word of tau-bar is cleared:
-          // what remains is a subnormal below 2.2e-314, whose products
-          // with chords (below 1e10 cm) stay below 3e-304 and vanish in
-          // the sums.  One select per product instead of two.
-          const int hi = __double2hiint(tb), lo = __double2loint(tb);
-#pragma unroll
-          for (int u = 0; u < kAdjointSegments; ++u)
-            sb[u] = fma(__hiloint2double(u <= k ? hi : 0, lo), ct[u], sb[u]);
-        }
-        tb = tb_next;
-        last = last_next;
-        t = t_next;
-      }
-#pragma unroll
-      for (int u = kAdjointSegments - 1; u >= 0; --u) {
-        const int q = qb + u;
-        if (q > L - 2) continue;
-        const double kb = sb[u] + s_hi;                              // d logL / d k_{q+1}
-        if (valid) kp[size_t(q + 1) * level_step + 2 * kKeptValue] = float(kb);
-        double x4[4] = {kb * sr, 0.0, 0.0, 0.0};
-        emitSums<4>(out + size_t(q + 1) * tiles * K, lane, x4, ns + 3, 1);
-        s_hi = sb[u];
-      }
+    for (int u = 0; u < kAdjointSegments; ++u) sb[u] = 0.0;
+    const int t_end = min(qb + kAdjointSegments, L - 1);
+    // this lane's tau-bar and last segment of path t, for the paths that
+    // reach the pass (the next one's are loaded while a path's products
+    // run); the others end below every segment of the pass
+    auto column = [&](int t) { return kp + size_t(t) * level_step; };
+    auto next = [&](int t) {                         // the first path from t on that reaches the pass
+      while (t < t_end && rl[t] < qb) ++t;
+      return t;
+    };
+    int t = next(0);
+    double tb = 0.0;
+    int last = -1;
+    if (t < t_end) {
+      tb = double(column(t)[kKeptValue]);
+      last = int(column(t)[2 * kKeptValue]);
     }
-    {
-      const double kb = s_hi;                                        // d logL / d k_0
-      if (valid) kp[2 * kKeptValue] = float(kb);
+    while (t < t_end) {
+      const int t_next = next(t + 1);
+      double tb_next = 0.0;
+      int last_next = -1;
+      if (t_next < t_end) {                          // uniform
+        tb_next = double(column(t_next)[kKeptValue]);
+        last_next = int(column(t_next)[2 * kKeptValue]);
+      }
+      {
+        const double* ct = c + size_t(t) * rows + qb;
+        const int k = last - qb;                     // this lane sums segments qb .. qb + k
+        // Past segment qb + k only the high word of tau-bar is cleared:
+        // what remains is a subnormal below 2.2e-314, whose products
+        // with chords (below 1e10 cm) stay below 3e-304 and vanish in
+        // the sums.  One select per product instead of two.
+        const int hi = __double2hiint(tb), lo = __double2loint(tb);
+#pragma unroll
+        for (int u = 0; u < kAdjointSegments; ++u)
+          sb[u] = fma(__hiloint2double(u <= k ? hi : 0, lo), ct[u], sb[u]);
+      }
+      tb = tb_next;
+      last = last_next;
+      t = t_next;
+    }
+#pragma unroll
+    for (int u = kAdjointSegments - 1; u >= 0; --u) {
+      const int q = qb + u;
+      if (q > L - 2) continue;
+      const double kb = sb[u] + s_hi;                              // d logL / d k_{q+1}
+      if (valid) kp[size_t(q + 1) * level_step + 2 * kKeptValue] = float(kb);
       double x4[4] = {kb * sr, 0.0, 0.0, 0.0};
-      emitSums<4>(out, lane, x4, ns + 3, 1);
+      emitSums<4>(out + size_t(q + 1) * tiles * K, lane, x4, ns + 3, 1);
+      s_hi = sb[u];
     }
+  }
+  {
+    const double kb = s_hi;                                        // d logL / d k_0
+    if (valid) kp[2 * kKeptValue] = float(kb);
+    double x4[4] = {kb * sr, 0.0, 0.0, 0.0};
+    emitSums<4>(out, lane, x4, ns + 3, 1);
   }
 }
 
@@ -979,24 +1017,25 @@ __global__ __launch_bounds__(kWave) void segmentAdjointKernel(Records rec, const
 // every window is done.  chord_t (chordTransposeKernel) is made before the
 // first window.
 template <int NS>
-void launchTransmissionAdjoint(dim3 grid, dim3 rt_grid, hipStream_t s, const double* tables, size_t stride,
+void launchTransmissionAdjoint(hipStream_t s, const double* tables, size_t stride,
                                const double* rayleigh, Records rec, int L, int n, int tiles, TileWindow win,
                                int batch, const double* fbar, const double* depth, float* keep, double* partial,
                                int ranges, int r0, int r1, int nu_per_range, double* chord_partial,
                                const double* chord_t, int* reach, const double* hminus, int kslots) {
-  hipLaunchKernelGGL(tangentAdjointKernel, rt_grid, dim3(kWave), 0, s, rec, L, n, stride, tiles, win, batch, NS,
+  const dim3 items(unsigned(nbItems(win.count, batch)));
+  hipLaunchKernelGGL(tangentAdjointKernel, items, dim3(kWave), 0, s, rec, L, n, stride, tiles, win, batch, NS,
                      kslots, fbar, depth, keep, partial);
   const int P = L - 1, blocks = (P + kChordBlock - 1) / kChordBlock;
   hipLaunchKernelGGL(chordAdjointKernel,
                      dim3(unsigned(blocks * (blocks + 1) / 2), unsigned(batch), unsigned(r1 - r0)), dim3(256), 0, s,
                      keep, L, n, stride, ranges, r0, nu_per_range, win, tiles, reach, chord_partial);
-  hipLaunchKernelGGL(segmentAdjointKernel, rt_grid, dim3(kWave), 0, s, rec, chord_t, rayleigh, L, n, stride, tiles,
+  hipLaunchKernelGGL(segmentAdjointKernel, items, dim3(kWave), 0, s, rec, chord_t, rayleigh, L, n, stride, tiles,
                      win, batch, NS, kslots, keep, partial, reach);
   if (hminus)
-    hipLaunchKernelGGL((opacityAdjointKernel<NS, true>), grid, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
+    hipLaunchKernelGGL((opacityAdjointKernel<NS, true>), items, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles,
                        win, batch, keep, hminus, kslots, partial);
   else
-    hipLaunchKernelGGL(opacityAdjointKernel<NS>, grid, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles, win,
+    hipLaunchKernelGGL(opacityAdjointKernel<NS>, items, dim3(kWave), 0, s, tables, stride, rec, L, n, tiles, win,
                        batch, keep, hminus, kslots, partial);
 }
 
@@ -1032,7 +1071,6 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
             K = int(adjointSlots(NS, hminus_, cloud_models_ > 0));
   const int tiles = (n + kWave - 1) / kWave;
   const int grid = int(align8(std::max<size_t>(8, size_t(nb_cus_) * kAdjointWavesPerCu)));
-  const int rt_grid = int(align8(std::max<size_t>(8, size_t(nb_cus_) * kRtWavesPerCu)));
 
   // points per chunk: kept forward quantities within the budget (and 80 % of
   // the free memory, checked when the buffers grow), else recomputed
@@ -1183,7 +1221,7 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
           launchBatchSpectrum(ModelKind::transmission, 1, launch, first, keep, nu_first, nu_end - nu_first, reach);
         }
         withSlots(species_stride_, [&](auto ns) {
-          launchTransmissionAdjoint<ns>(dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, tables_, stride_, rayleigh_,
+          launchTransmissionAdjoint<ns>(s, tables_, stride_, rayleigh_,
                                         rec, L, n, tiles, win, cb, adj_fbar_, batch_flux_ + first * stride_, keep,
                                         adj_partial_, ranges, r0, r1, nu_per_range, chord_partial, chord_t, reach,
                                         hminus_, K);
@@ -1198,7 +1236,7 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
             "read chord gradients");
     } else {
       withSlots(species_stride_, [&](auto ns) {
-        launchAdjoint<ns>(kept, dim3(unsigned(grid)), dim3(unsigned(rt_grid)), s, wavenumber_, wavelength_, tables_,
+        launchAdjoint<ns>(kept, dim3(unsigned(grid)), s, wavenumber_, wavelength_, tables_,
                           stride_, rec, L, n, tiles, cb, adj_fbar_, adj_intensity_, adj_partial_, hminus_, K,
                           cloud_slot0);
       });

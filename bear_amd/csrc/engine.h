@@ -58,10 +58,11 @@ struct alignas(64) LevelState {
   // exponential table (exp_table.h): w x 128, tableDensity(log2 n)
   double table_w[2][4];
   double table_n[16];
-  // per stencil group the fractions between its temperature rows and, where
-  // every temperature row has the same pressures, between its pressure rows
-  // (isothermal stencils, Opacity64Isothermal)
-  double fraction_t[2], fraction_p[2];
+  // per stencil group the fractions of the interpolation: between its
+  // temperature rows, with the derivative by T, and between the pressure rows
+  // of the lower and the upper temperature (the isothermal stencils, whose
+  // two are the same, and the adjoint)
+  double fraction_t[2], slope_t[2], fraction_p[2], fraction_q[2];
   // the weights and densities for the reduced-precision tables (LevelSpecies32 values)
   float group_w32[2][4];
   float log2_n32[16];

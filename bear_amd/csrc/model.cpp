@@ -139,7 +139,9 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       group_st[g] = st;
       const double ft = st.f_t, fl = st.f_p_lower, fu = st.f_p_upper;
       lev[l].fraction_t[g] = ft;
+      lev[l].slope_t[g] = st.dft;
       lev[l].fraction_p[g] = fl;
+      lev[l].fraction_q[g] = fu;
       lev[l].group_w[g][0] = (1.0 - ft) * (1.0 - fl) * log2_ten;
       lev[l].group_w[g][1] = (1.0 - ft) * fl * log2_ten;
       lev[l].group_w[g][2] = ft * (1.0 - fu) * log2_ten;

@@ -236,7 +236,9 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       gst[q] = st;
       const double ft = st.f_t, fl = st.f_p_lower, fu = st.f_p_upper;
       ls.fraction_t[q] = ft;
+      ls.slope_t[q] = st.dft;
       ls.fraction_p[q] = fl;
+      ls.fraction_q[q] = fu;
       ls.group_w[q][0] = (1.0 - ft) * (1.0 - fl) * kLog2Ten;
       ls.group_w[q][1] = (1.0 - ft) * fl * kLog2Ten;
       ls.group_w[q][2] = ft * (1.0 - fu) * kLog2Ten;
