@@ -32,7 +32,7 @@ void deviceFree(void* p) {
   if (p) (void)hipFree(p);
 }
 
-constexpr int kStageBlock = 256;
+constexpr int kStageBlock = 512;
 constexpr double kLog2Ten = 3.321928094887362347870319429489390175864831393;
 constexpr double kBoltzmann = 1.3806504e-16;     // cgs, as the host's phys::boltzmann_k
 constexpr double kGas = 8.314472e7;              // phys::gas_constant
@@ -56,16 +56,14 @@ struct DeviceStencil {
 __device__ DeviceStencil bracket(const StagePlan& P, const unsigned char* blob, int g, int l, double t) {
   const StageGrid G = at<StageGrid>(blob, P.grids)[g];
   const double* tn = at<double>(blob, P.grid_t) + G.t_offset;       // each temperature row's temperature
-  int lo = 0, hi = 0;
-  if (t < tn[0]) {
-  } else if (t > tn[G.nt - 1]) {
-    lo = hi = G.nt - 1;
-  } else {
-    for (int i = 0; i < G.nt; ++i) {
-      if (tn[i] == t) { lo = hi = i; break; }
-      if (tn[i] < t && tn[i + 1] > t) { lo = i; hi = i + 1; break; }
-    }
-  }
+  // the rows are in increasing temperature: t is at or above the first `upto`
+  // of them (counted without a branch, so that the loads do not wait for one
+  // another)
+  int upto = 0;
+#pragma unroll 8
+  for (int i = 0; i < G.nt; ++i) upto += tn[i] <= t ? 1 : 0;
+  const int lo = max(upto - 1, 0);
+  const int hi = (upto == 0 || upto == G.nt || tn[lo] == t) ? lo : lo + 1;
   const StagePick* picks = at<StagePick>(blob, P.picks) + G.picks_offset + size_t(l) * G.nt;
   const StagePick pl = picks[lo], ph = picks[hi];
   const int* tstart = at<int>(blob, P.grid_tstart) + G.tstart_offset;
@@ -87,16 +85,21 @@ __device__ DeviceStencil bracket(const StagePlan& P, const unsigned char* blob, 
   return s;
 }
 
-__device__ __forceinline__ uint32_t rowId(const StagePlan& P, const unsigned char* blob, const StageSpecies& sp,
-                                          int t_pos, int p_pos) {
-  const StageGrid G = at<StageGrid>(blob, P.grids)[sp.grid];
-  const int t0 = at<int>(blob, P.grid_tstart)[G.tstart_offset + t_pos];
-  return at<uint32_t>(blob, P.row_ids)[sp.row_offset + t0 + p_pos];
+// offset of row p_pos of temperature row t_pos within its species' rows
+__device__ __forceinline__ uint32_t rowOffset(const StagePlan& P, const unsigned char* blob, int g, int t_pos,
+                                              int p_pos) {
+  const StageGrid G = at<StageGrid>(blob, P.grids)[g];
+  return uint32_t(at<int>(blob, P.grid_tstart)[G.tstart_offset + t_pos] + p_pos);
 }
 
 // One workgroup per live point.  LDS: per level the temperature, total
 // density, mean molecular weight, density rho and altitude, then the active
 // species' densities [L][nb_active] and the temperature degrees of freedom.
+// A batch has a workgroup or less per CU, so latencies bound it, one after
+// the other: what is serial over the levels is the altitudes' additions alone,
+// and the slots of a level are staged by different threads (with one thread
+// per level: 16 points of 40 levels and 3 absorbers 38 us, now 19; 64 points
+// of 100 levels and 6 absorbers 76 us, now 55).
 __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const unsigned char* __restrict__ blob,
                                                            const double* __restrict__ params, int batch,
                                                            unsigned char* __restrict__ records, size_t rec_bytes,
@@ -127,6 +130,12 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       dof[0] = tp[0];
       for (int i = 1; i < P.nb_temp; ++i) dof[i] = dof[i - 1] * tp[i];
     }
+  }
+  unsigned char* rec = records + size_t(m) * rec_bytes;
+  LevelState* lev = reinterpret_cast<LevelState*>(rec + rec_levels);
+  {
+    uint64_t* w = reinterpret_cast<uint64_t*>(lev);
+    for (size_t q = size_t(tid); q < size_t(L) * (sizeof(LevelState) / 8); q += kStageBlock) w[q] = 0;
   }
   __syncthreads();
 
@@ -187,38 +196,80 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
   if (neg) atomicOr(&s_neglect, 1);
   __syncthreads();
 
-  // altitudes (atmosphere.cpp:288-350), in order over the levels
+  // altitudes (atmosphere.cpp:288-350): the increments at the point's gravity
+  // side by side, then their sum in order over the levels
+  const bool scale_height = P.alt_kind == 2 && p[3] > 0;
   const double g = pow(10.0, p[0]);
-  if (tid == 0) {
-    z[0] = 0.0;
-    if (P.alt_kind == 2 && p[3] > 0) {
-      const double h = p[3] * 100000.0;
-      const double* lr = at<double>(blob, P.log_ratio);
-      for (int l = 1; l < L; ++l) z[l] = -h * lr[l];
-    } else {
-      const double radius = p[1];
-      for (int l = 1; l < L; ++l) {
-        double gl = g;
-        if (P.variable_gravity) {
-          const double x = radius / (radius + z[l - 1]);
-          gl = g * (x * x);
-        }
-        z[l] = z[l - 1] + (1.0 / (rho[l] * gl) + 1.0 / (rho[l - 1] * gl)) * 0.5 * (pres[l - 1] * 1e6 - pres[l] * 1e6);
+  for (int l = tid; l < L; l += kStageBlock) {
+    double step = 0.0;
+    if (l > 0) {
+      if (scale_height)
+        step = -(p[3] * 100000.0) * at<double>(blob, P.log_ratio)[l];          // the altitude itself
+      else
+        step = (1.0 / (rho[l] * g) + 1.0 / (rho[l - 1] * g)) * 0.5 * (pres[l - 1] * 1e6 - pres[l] * 1e6);
+    }
+    z[l] = step;
+  }
+  __syncthreads();
+  if (tid == 0 && !scale_height) {
+    // g falls off as (radius / (radius + z))^2, with z of the level below
+    const double falloff = P.variable_gravity ? 1.0 / p[1] : 0.0;
+    double sum = 0.0;
+    constexpr int kAhead = 8;                       // increments read ahead of the sums
+    for (int l0 = 0; l0 < L; l0 += kAhead) {
+      double step[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) step[k] = z[min(l0 + k, L - 1)];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const double x = fma(sum, falloff, 1.0);
+        sum = fma(step[k], x * x, sum);
+        if (l0 + k < L) z[l0 + k] = sum;
       }
+    }
+  }
+  // meanwhile another wavefront: the point's scalars and observation shifts
+  // (emission.cpp:108-120, secondary_eclipse.cpp:117-153,
+  // transmission.cpp:150-195, forward_model.cpp:184-204, retrieval.cpp:333-336)
+  if (tid / 64 == 1) {
+    const int lane = tid & 63;
+    double hottest = T[0];
+    for (int l = lane; l < L; l += 64) hottest = fmax(hottest, T[l]);
+    for (int o = 32; o > 0; o >>= 1) hottest = fmax(hottest, __shfl_xor(hottest, o, 64));
+    if (lane == 0) {
+      BatchModel& bm = *reinterpret_cast<BatchModel*>(rec);
+      bm = BatchModel{};
+      if (P.kind == int(ModelKind::emission)) {
+        const double sc = kJupiter / p[2];
+        bm.scaling = sc * sc * p[1];
+      } else if (P.kind == int(ModelKind::eclipse)) {
+        bm.scaling = 1.0;
+        bm.star_inv_temperature = 1.0 / p[2];
+        bm.depth_scale = p[1] * p[1] * 1e6;
+      } else {
+        bm.bottom_radius = p[1];
+        bm.star_radius = p[2];
+      }
+      bm.min_inv_temperature = 1.0 / hottest;
+      bm.inflation = P.error_inflation ? pow(10.0, p[P.nb_params - 1]) : 0.0;
+      double* shifts = reinterpret_cast<double*>(rec + rec_shifts);
+      const int* om = at<int>(blob, P.obs_mods);
+      int k = 0;
+      for (int o = 0; o < P.nb_obs; ++o) {
+        shifts[o] = om[o] ? p[P.mods_offset + k] : 0.0;
+        k += om[o];
+      }
+      neglect[m] = s_neglect;
     }
   }
   __syncthreads();
 
-  // per level: LevelState and the stencils of every slot (stageLevels)
-  unsigned char* rec = records + size_t(m) * rec_bytes;
-  LevelState* lev = reinterpret_cast<LevelState*>(rec + rec_levels);
+  // per level: LevelState and the two groups' stencils (stageLevels).  The
+  // groups' row offsets go over the level's T, ntot, mmw and rho, which no
+  // other thread reads from here on.
   const StageSpecies* sps = at<StageSpecies>(blob, P.species);
   for (int l = tid; l < L; l += kStageBlock) {
     LevelState& ls = lev[l];
-    {
-      uint64_t* w = reinterpret_cast<uint64_t*>(&ls);
-      for (size_t q = 0; q < sizeof(LevelState) / 8; ++q) w[q] = 0;
-    }
     const double t = T[l];
     const double* n = nd + size_t(l) * NA;
     ls.temperature = t;
@@ -229,11 +280,17 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       ls.cloud_scale = P.kind == int(ModelKind::transmission) ? 1.0 / (z[l] - z[l - 1]) : 1.0;
       ls.half_dz = (z[l] - z[l - 1]) * 0.5;
     }
-    DeviceStencil gst[2];
+#pragma unroll
     for (int q = 0; q < 2; ++q) {
       if (P.group_grid[q] < 0) continue;
       const DeviceStencil st = bracket(P, blob, P.group_grid[q], l, t);
-      gst[q] = st;
+      if (P.grouped) {
+        uint32_t row[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) row[k] = rowOffset(P, blob, P.group_grid[q], st.t_pos[k / 2], st.p_pos[k]);
+        sh[2 * q * L + l] = __hiloint2double(int(row[1]), int(row[0]));        // T, mmw
+        sh[(2 * q + 1) * L + l] = __hiloint2double(int(row[3]), int(row[2]));  // ntot, rho
+      }
       const double ft = st.f_t, fl = st.f_p_lower, fu = st.f_p_upper;
       ls.fraction_t[q] = ft;
       ls.slope_t[q] = st.dft;
@@ -253,113 +310,107 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       ls.group_u[q][2] = (1.0 - fu) * du;
       ls.group_u[q][3] = fu * du;
     }
-    uint32_t absorbers = 0;
-    for (int s = 0; s < P.NS; ++s) {
-      double dens = 0.0;
-      DeviceStencil st{{0, 0}, {0, 0, 0, 0}, 0.0, 0.0, 0.0, 0.0};
-      uint32_t row[4] = {0, 0, 0, 0};
-      if (s < P.S) {
-        const StageSpecies sp = sps[s];
-        dens = slot[sp.species_id] >= 0 ? n[slot[sp.species_id]] : 0.0;       // opacity_species.cpp:407-412
-        if (sp.partner0 >= 0) dens *= slot[sp.partner0] >= 0 ? n[slot[sp.partner0]] : 0.0;
-        if (sp.partner1 >= 0) dens *= slot[sp.partner1] >= 0 ? n[slot[sp.partner1]] : 0.0;
-        if (dens != 0) ++absorbers;
-        st = P.grouped ? gst[(P.group1 >> s) & 1u] : bracket(P, blob, sp.grid, l, t);
-        for (int k = 0; k < 4; ++k) row[k] = rowId(P, blob, sp, st.t_pos[k / 2], st.p_pos[k]);
-      }
-      uint32_t block[4];
-      for (int k = 0; k < 4; ++k) block[k] = uint32_t(row[k] * P.blocks_per_row);
-      const double ft = st.f_t, fl = st.f_p_lower, fu = st.f_p_upper;
-      if (wide) {
-        LevelSpecies& d = reinterpret_cast<LevelSpecies*>(rec + rec_species)[size_t(l) * P.NS + s];
-        d.w[0] = (1.0 - ft) * (1.0 - fl) * kLog2Ten;
-        d.w[1] = (1.0 - ft) * fl * kLog2Ten;
-        d.w[2] = ft * (1.0 - fu) * kLog2Ten;
-        d.w[3] = ft * fu * kLog2Ten;
-        d.log2_n = dens > 0 ? log2(dens) : kZeroDensityLog2;
-        if (s < 16) {
-          ls.log2_n[s] = d.log2_n;
-          ls.table_n[s] = tableDensity(d.log2_n);
-        }
-        for (int k = 0; k < 4; ++k) d.block[k] = block[k];
-        d.reload = 0;
-        d.pad = 0;
-        LevelSpeciesAdjoint& a = reinterpret_cast<LevelSpeciesAdjoint*>(rec + rec_adjoint)[size_t(l) * P.NS + s];
-        const double du = st.dft * kLog2Ten;
-        a.u[0] = -(1.0 - fl) * du;
-        a.u[1] = -fl * du;
-        a.u[2] = (1.0 - fu) * du;
-        a.u[3] = fu * du;
-        for (int k = 0; k < 4; ++k) a.pad[k] = 0.0;
-      } else {
-        LevelSpecies32& d = reinterpret_cast<LevelSpecies32*>(rec + rec_species)[size_t(l) * P.NS + s];
-        d.w[0] = float((1.0 - ft) * (1.0 - fl) * kLog2Ten);
-        d.w[1] = float((1.0 - ft) * fl * kLog2Ten);
-        d.w[2] = float(ft * (1.0 - fu) * kLog2Ten);
-        d.w[3] = float(ft * fu * kLog2Ten);
-        d.log2_n = dens > 0 ? float(log2(dens)) : -__builtin_huge_valf();
-        if (s < 16) ls.log2_n32[s] = d.log2_n;
-        for (int k = 0; k < 4; ++k) d.block[k] = block[k];
-        d.reload = 0;
-        d.pad[0] = d.pad[1] = 0;
-      }
-    }
-    ls.absorbers = absorbers;
   }
   __syncthreads();
+  // from here z holds two words per level: the slots whose rows changed (bit
+  // per slot) and the number of slots of non-zero density
+  uint32_t* words = reinterpret_cast<uint32_t*>(z);
+  for (int l = tid; l < 2 * L; l += kStageBlock) words[l] = 0;
+  __syncthreads();
 
-  // reload flags: a slot's rows differ from the previous level's (always at level 0)
-  for (int l = tid; l < L; l += kStageBlock) {
-    uint32_t bits = 0;
-    for (int s = 0; s < P.NS; ++s) {
-      uint32_t changed = l == 0;
-      const size_t e = size_t(l) * P.NS + s;
-      if (wide) {
-        LevelSpecies* d = reinterpret_cast<LevelSpecies*>(rec + rec_species);
-        if (l > 0)
-          for (int k = 0; k < 4; ++k) changed |= d[e - P.NS].block[k] != d[e].block[k];
-        d[e].reload = changed;
+  // per slot of a level: its density, rows and weights, and whether its rows
+  // differ from the previous level's (always at level 0)
+  for (int e = tid; e < L * P.NS; e += kStageBlock) {
+    const int l = e / P.NS, s = e - l * P.NS;
+    LevelState& ls = lev[l];
+    double dens = 0.0, ft = 0.0, fl = 0.0, fu = 0.0, dft = 0.0;
+    uint32_t block[4] = {0, 0, 0, 0};
+    uint32_t changed = l == 0;
+    if (s < P.S) {
+      const StageSpecies sp = sps[s];
+      const double* n = nd + size_t(l) * NA;
+      dens = slot[sp.species_id] >= 0 ? n[slot[sp.species_id]] : 0.0;         // opacity_species.cpp:407-412
+      if (sp.partner0 >= 0) dens *= slot[sp.partner0] >= 0 ? n[slot[sp.partner0]] : 0.0;
+      if (sp.partner1 >= 0) dens *= slot[sp.partner1] >= 0 ? n[slot[sp.partner1]] : 0.0;
+      const uint32_t* ids = at<uint32_t>(blob, P.row_ids) + sp.row_offset;
+      const int q = int((P.group1 >> s) & 1u);
+      auto rows = [&](int level, const DeviceStencil* st, uint32_t (&row)[4]) {
+        if (P.grouped) {
+          const double a = sh[2 * q * L + level], b = sh[(2 * q + 1) * L + level];
+          row[0] = ids[__double2loint(a)];
+          row[1] = ids[__double2hiint(a)];
+          row[2] = ids[__double2loint(b)];
+          row[3] = ids[__double2hiint(b)];
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) row[k] = ids[rowOffset(P, blob, sp.grid, st->t_pos[k / 2], st->p_pos[k])];
+        }
+      };
+      DeviceStencil st;
+      if (P.grouped) {
+        ft = ls.fraction_t[q];
+        dft = ls.slope_t[q];
+        fl = ls.fraction_p[q];
+        fu = ls.fraction_q[q];
       } else {
-        LevelSpecies32* d = reinterpret_cast<LevelSpecies32*>(rec + rec_species);
-        if (l > 0)
-          for (int k = 0; k < 4; ++k) changed |= d[e - P.NS].block[k] != d[e].block[k];
-        d[e].reload = changed;
+        st = bracket(P, blob, sp.grid, l, T[l]);
+        ft = st.f_t;
+        dft = st.dft;
+        fl = st.f_p_lower;
+        fu = st.f_p_upper;
       }
-      bits |= changed << s;
+      uint32_t row[4], below[4];
+      rows(l, &st, row);
+      if (l > 0) {
+        if (!P.grouped) st = bracket(P, blob, sp.grid, l - 1, T[l - 1]);
+        rows(l - 1, &st, below);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) changed |= row[k] != below[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) block[k] = uint32_t(row[k] * P.blocks_per_row);
     }
-    lev[l].reload = bits;
-    if (l > 0 && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
-  }
-
-  // the point's scalars and observation shifts (emission.cpp:108-120,
-  // secondary_eclipse.cpp:117-153, transmission.cpp:150-195,
-  // forward_model.cpp:184-204, retrieval.cpp:333-336)
-  if (tid == 0) {
-    BatchModel& bm = *reinterpret_cast<BatchModel*>(rec);
-    bm = BatchModel{};
-    if (P.kind == int(ModelKind::emission)) {
-      const double sc = kJupiter / p[2];
-      bm.scaling = sc * sc * p[1];
-    } else if (P.kind == int(ModelKind::eclipse)) {
-      bm.scaling = 1.0;
-      bm.star_inv_temperature = 1.0 / p[2];
-      bm.depth_scale = p[1] * p[1] * 1e6;
+    if (changed && s < 32) atomicOr(&words[2 * l], 1u << s);
+    if (dens != 0) atomicAdd(&words[2 * l + 1], 1u);
+    if (wide) {
+      LevelSpecies& d = reinterpret_cast<LevelSpecies*>(rec + rec_species)[e];
+      d.w[0] = (1.0 - ft) * (1.0 - fl) * kLog2Ten;
+      d.w[1] = (1.0 - ft) * fl * kLog2Ten;
+      d.w[2] = ft * (1.0 - fu) * kLog2Ten;
+      d.w[3] = ft * fu * kLog2Ten;
+      d.log2_n = dens > 0 ? log2(dens) : kZeroDensityLog2;
+      if (s < 16) {
+        ls.log2_n[s] = d.log2_n;
+        ls.table_n[s] = tableDensity(d.log2_n);
+      }
+      for (int k = 0; k < 4; ++k) d.block[k] = block[k];
+      d.reload = changed;
+      d.pad = 0;
+      LevelSpeciesAdjoint& a = reinterpret_cast<LevelSpeciesAdjoint*>(rec + rec_adjoint)[e];
+      const double du = dft * kLog2Ten;
+      a.u[0] = -(1.0 - fl) * du;
+      a.u[1] = -fl * du;
+      a.u[2] = (1.0 - fu) * du;
+      a.u[3] = fu * du;
+      for (int k = 0; k < 4; ++k) a.pad[k] = 0.0;
     } else {
-      bm.bottom_radius = p[1];
-      bm.star_radius = p[2];
+      LevelSpecies32& d = reinterpret_cast<LevelSpecies32*>(rec + rec_species)[e];
+      d.w[0] = float((1.0 - ft) * (1.0 - fl) * kLog2Ten);
+      d.w[1] = float((1.0 - ft) * fl * kLog2Ten);
+      d.w[2] = float(ft * (1.0 - fu) * kLog2Ten);
+      d.w[3] = float(ft * fu * kLog2Ten);
+      d.log2_n = dens > 0 ? float(log2(dens)) : -__builtin_huge_valf();
+      if (s < 16) ls.log2_n32[s] = d.log2_n;
+      for (int k = 0; k < 4; ++k) d.block[k] = block[k];
+      d.reload = changed;
+      d.pad[0] = d.pad[1] = 0;
     }
-    double hottest = T[0];
-    for (int l = 1; l < L; ++l) hottest = fmax(hottest, T[l]);
-    bm.min_inv_temperature = 1.0 / hottest;
-    bm.inflation = P.error_inflation ? pow(10.0, p[P.nb_params - 1]) : 0.0;
-    double* shifts = reinterpret_cast<double*>(rec + rec_shifts);
-    const int* om = at<int>(blob, P.obs_mods);
-    int k = 0;
-    for (int o = 0; o < P.nb_obs; ++o) {
-      shifts[o] = om[o] ? p[P.mods_offset + k] : 0.0;
-      k += om[o];
-    }
-    neglect[m] = s_neglect;
+  }
+  __syncthreads();
+  for (int l = tid; l < L; l += kStageBlock) {
+    lev[l].reload = words[2 * l];
+    lev[l].absorbers = words[2 * l + 1];
+    if (l > 0 && words[2 * l + 1] == 0 && words[2 * l - 1] == 0) lev[l].half_dz = 0.0;
   }
 }
 
