@@ -141,13 +141,16 @@ __global__ __launch_bounds__(1024) void sumBatchKernel(const double* __restrict_
 }
 
 // high-resolution output per point: emission F per micron, eclipse depth
-// F / F_* (Rp/Rs)^2 1e6, transmission depth
+// F / F_* (Rp/Rs)^2 1e6, transmission depth; elements [first, first + count)
+// of the [point][n] output to out (pinned host memory)
 __global__ __launch_bounds__(kBatchBlock) void batchSpectrumKernel(
     const double* __restrict__ flux, size_t stride, const double* __restrict__ wavenumber,
-    const double* __restrict__ wavelength, Records rec, int mode, int n, double* __restrict__ out) {
-  const int i = blockIdx.x * kBatchBlock + threadIdx.x;
-  const int m = blockIdx.y;
-  if (i >= n) return;
+    const double* __restrict__ wavelength, Records rec, int mode, int n, size_t first, int count,
+    double* __restrict__ out) {
+  const int k = int(blockIdx.x) * kBatchBlock + int(threadIdx.x);
+  if (k >= count) return;
+  const size_t m = (first + size_t(k)) / size_t(n);
+  const int i = int((first + size_t(k)) - m * size_t(n));
   const BatchModel* bm = reinterpret_cast<const BatchModel*>(rec.at(m));
   const double f = flux[size_t(m) * stride + i];
   double v = f;
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(kBatchBlock) void batchSpectrumKernel(
   } else if (mode == 1) {
     v = f * recip(starFlux(wavenumber[i], bm->star_inv_temperature)) * bm->depth_scale;
   }
-  out[size_t(m) * n + i] = v;
+  out[k] = v;
 }
 
 size_t align(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -522,32 +525,20 @@ void DeviceEngine::evaluateBatch(ModelKind kind, size_t batch, bool staged) {
 }
 
 void DeviceEngine::copyBatchBins(size_t batch, std::vector<double>& out) {
-  hipStream_t s = static_cast<hipStream_t>(stream_);
   out.resize(batch * n_bins_);
-  if (!out.empty())
-    check(hipMemcpyAsync(out.data(), batch_bins_, out.size() * sizeof(double), hipMemcpyDeviceToHost, s),
-          "read batch bins");
-  check(hipStreamSynchronize(s), "read batch bins");
+  copyDoubles(out.data(), batch_bins_, out.size());
 }
 
 void DeviceEngine::copyBatchSpectrum(ModelKind kind, size_t batch, double* host) {
   hipStream_t s = static_cast<hipStream_t>(stream_);
   const Records rec{batch_dev_, rec_bytes_, rec_levels_, rec_species_, rec_adjoint_, rec_shifts_, groups_};
-  const int n = int(n_points_);
-  double* out = deviceAlloc<double>(batch * n_points_, "batch spectrum output");
-  try {
-    hipLaunchKernelGGL(batchSpectrumKernel, dim3(unsigned((n + kBatchBlock - 1) / kBatchBlock), unsigned(batch)),
-                       dim3(kBatchBlock), 0, s, batch_flux_, stride_, wavenumber_, wavelength_, rec,
-                       kind == ModelKind::emission ? 0 : (kind == ModelKind::eclipse ? 1 : 2), n, out);
+  const int n = int(n_points_), mode = kind == ModelKind::emission ? 0 : (kind == ModelKind::eclipse ? 1 : 2);
+  streamOut(batch * n_points_, host, [&](size_t first, size_t count, double* out) {
+    hipLaunchKernelGGL(batchSpectrumKernel, dim3(unsigned((count + kBatchBlock - 1) / kBatchBlock)),
+                       dim3(kBatchBlock), 0, s, batch_flux_, stride_, wavenumber_, wavelength_, rec, mode, n, first,
+                       int(count), out);
     check(hipGetLastError(), "batch spectrum kernel");
-    check(hipMemcpyAsync(host, out, batch * n_points_ * sizeof(double), hipMemcpyDeviceToHost, s),
-          "read batch spectrum");
-    check(hipStreamSynchronize(s), "read batch spectrum");
-  } catch (...) {
-    deviceFree(out);
-    throw;
-  }
-  deviceFree(out);
+  });
 }
 
 void DeviceEngine::releaseBatch() {

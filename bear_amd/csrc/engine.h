@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <type_traits>
 #include <vector>
 
@@ -502,6 +503,13 @@ class DeviceEngine {
   double* ll_host_dev_ = nullptr;                // ll_host_ as the device addresses it
   // measurement
   bool profiling_ = false, event_pending_ = false;
+  // host[0, count) in pieces of a pinned ring: produce(first, length, out)
+  // enqueues the writing of elements [first, first + length) to out
+  void streamOut(size_t count, double* host, const std::function<void(size_t, size_t, double*)>& produce);
+  void copyDoubles(double* host, const double* dev, size_t n);   // and waits for the stream
+  static constexpr size_t kOutPiece = size_t(1) << 17, kOutPieces = 4;     // doubles: 4 MiB together
+  double* out_host_ = nullptr;
+  void* out_events_[kOutPieces] = {nullptr, nullptr, nullptr, nullptr};
   void* event_start_ = nullptr;
   void* event_stop_ = nullptr;
   size_t timed_launches_ = 0, distinct_rows_ = 0;

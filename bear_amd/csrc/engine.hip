@@ -373,6 +373,9 @@ DeviceEngine::~DeviceEngine() {
                   (void*)star_})
     deviceFree(p);
   if (staging_host_) (void)hipHostFree(staging_host_);
+  if (out_host_) (void)hipHostFree(out_host_);
+  for (void* e : out_events_)
+    if (e) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
   if (event_start_) (void)hipEventDestroy(static_cast<hipEvent_t>(event_start_));
   if (event_stop_) (void)hipEventDestroy(static_cast<hipEvent_t>(event_stop_));
   if (stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(stream_));
@@ -812,10 +815,51 @@ void DeviceEngine::uploadStellarSpectrum(const std::vector<double>& flux) {
   check(hipStreamSynchronize(s), "copy stellar spectrum");
 }
 
-void DeviceEngine::copyFlux(double* host) {
+// A copy into memory that is not pinned goes through the runtime's own pinned
+// pieces, each waited for and copied by one thread in turn (13 spectra of
+// 45,000 wavenumbers, 4.7 MB: 430 us for 90 us of transfer).  Here the pieces
+// of the ring are written while an earlier one is copied on, by several
+// threads.
+void DeviceEngine::streamOut(size_t count, double* host,
+                             const std::function<void(size_t, size_t, double*)>& produce) {
+  check(hipSetDevice(device_), "hipSetDevice");
   hipStream_t s = static_cast<hipStream_t>(stream_);
-  check(hipMemcpyAsync(host, buffers().flux, n_points_ * sizeof(double), hipMemcpyDeviceToHost, s), "read flux");
-  check(hipStreamSynchronize(s), "evaluation");
+  if (!out_host_) {
+    void* h = nullptr;
+    check(hipHostMalloc(&h, kOutPieces * kOutPiece * sizeof(double), hipHostMallocDefault), "pinned output");
+    out_host_ = static_cast<double*>(h);
+  }
+  for (void*& e : out_events_)
+    if (!e) {
+      hipEvent_t event = nullptr;
+      check(hipEventCreateWithFlags(&event, hipEventDisableTiming), "hipEventCreate");
+      e = event;
+    }
+  const size_t pieces = (count + kOutPiece - 1) / kOutPiece;
+  auto length = [&](size_t k) { return std::min(kOutPiece, count - k * kOutPiece); };
+  auto start = [&](size_t k) {
+    produce(k * kOutPiece, length(k), out_host_ + k % kOutPieces * kOutPiece);
+    check(hipEventRecord(static_cast<hipEvent_t>(out_events_[k % kOutPieces]), s), "hipEventRecord");
+  };
+  for (size_t k = 0; k < std::min(pieces, kOutPieces); ++k) start(k);
+  for (size_t k = 0; k < pieces; ++k) {
+    check(hipEventSynchronize(static_cast<hipEvent_t>(out_events_[k % kOutPieces])), "read spectrum");
+    copyOut(host + k * kOutPiece, out_host_ + k % kOutPieces * kOutPiece, length(k));
+    if (k + kOutPieces < pieces) start(k + kOutPieces);
+  }
+}
+
+void DeviceEngine::copyDoubles(double* host, const double* dev, size_t n) {
+  streamOut(n, host, [&](size_t first, size_t count, double* out) {
+    check(hipMemcpyAsync(out, dev + first, count * sizeof(double), hipMemcpyDeviceToHost,
+                         static_cast<hipStream_t>(stream_)),
+          "read results");
+  });
+  if (n == 0) check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "evaluation");
+}
+
+void DeviceEngine::copyFlux(double* host) {
+  copyDoubles(host, buffers().flux, n_points_);
   collectTiming();
 }
 
@@ -867,17 +911,13 @@ double DeviceEngine::logLikelihood() {
 }
 
 void DeviceEngine::copyBins(std::vector<double>& out) {
-  hipStream_t s = static_cast<hipStream_t>(stream_);
   out.resize(n_bins_);
-  if (n_bins_) check(hipMemcpyAsync(out.data(), bins_, n_bins_ * sizeof(double), hipMemcpyDeviceToHost, s), "read bins");
-  check(hipStreamSynchronize(s), "evaluation");
+  copyDoubles(out.data(), bins_, n_bins_);
   collectTiming();
 }
 
 void DeviceEngine::copySpectrum(double* host, const double* spectrum_dev) {
-  hipStream_t s = static_cast<hipStream_t>(stream_);
-  check(hipMemcpyAsync(host, spectrum_dev, n_points_ * sizeof(double), hipMemcpyDeviceToHost, s), "read spectrum");
-  check(hipStreamSynchronize(s), "evaluation");
+  copyDoubles(host, spectrum_dev, n_points_);
 }
 
 double* DeviceEngine::spectrumBuffer() {

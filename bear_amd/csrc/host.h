@@ -21,6 +21,10 @@ struct Error : std::runtime_error {
 };
 [[noreturn]] void raise(int code, const std::string& msg);
 
+// dst[0, n) = src[0, n) by several threads where there is enough to copy (the
+// pages of a new dst are then also touched by several)
+void copyOut(double* dst, const double* src, size_t n);
+
 constexpr int kInvalidInput = -1, kFileNotFound = -2, kDevice = -3, kOutOfMemory = -4, kInternal = -5;
 
 // ------------------------------------------------------------------ constants

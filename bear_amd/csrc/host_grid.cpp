@@ -1,6 +1,9 @@
 // Spectral grid and species table of the host side.
+#include <omp.h>
+
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <fstream>
 #include <functional>
 
@@ -176,6 +179,21 @@ void SpectralGrid::sample(std::vector<ObservationSetup>& observations) {
     }
     o.range_index[0] = nearest(1.0 / o.range_wavelength[0] * 1e4, wavenumber, 0);
     o.range_index[1] = nearest(1.0 / o.range_wavelength[1] * 1e4, wavenumber, 0);
+  }
+}
+
+void copyOut(double* dst, const double* src, size_t n) {
+  constexpr size_t kShare = 8192;                          // doubles per thread at least: 64 KiB, some 10 us
+  const int threads = int(std::min<size_t>(8, std::min(size_t(omp_get_max_threads()), n / kShare)));
+  if (threads <= 1) {
+    std::memcpy(dst, src, n * sizeof(double));
+    return;
+  }
+  #pragma omp parallel num_threads(threads)
+  {
+    const size_t share = (n + size_t(omp_get_num_threads()) - 1) / size_t(omp_get_num_threads());
+    const size_t first = std::min(n, share * size_t(omp_get_thread_num()));
+    std::memcpy(dst + first, src + first, std::min(share, n - first) * sizeof(double));
   }
 }
 
