@@ -88,15 +88,10 @@ __global__ __launch_bounds__(kBatchBlock) void splitTableKernel(const double* __
   }
 }
 
-// Chord lengths of every point, transposed (chord[point][q][t], zero for
-// q < t and in the padding): sqrt((R+z_{q+1})^2 - (R+z_t)^2) -
-// sqrt((R+z_q)^2 - (R+z_t)^2), q >= t (transmission_spectrum.cpp:117-118,
-// 145-154); one workgroup per (segment q, point), FP64 and/or FP32.
-// Evaluated without contraction, as the host does: fused, a*a - b*b at a == b
-// leaves the rounding error of b*b, which can be negative.
+// Chord lengths of every point, transposed (chord[point][q][t], chordLength);
+// one workgroup per (segment q, point), FP64 and/or FP32.
 __global__ __launch_bounds__(kBatchBlock) void chordKernel(Records rec, int nb_levels, double* __restrict__ chord,
                                                            float* __restrict__ chord32) {
-#pragma clang fp contract(off)
   const int q = blockIdx.x, m = blockIdx.y;
   const int tangents = chordTangents(nb_levels);
   const unsigned char* r = rec.at(m);
@@ -104,12 +99,7 @@ __global__ __launch_bounds__(kBatchBlock) void chordKernel(Records rec, int nb_l
   const LevelState* levels = reinterpret_cast<const LevelState*>(r + rec.levels);
   const size_t row = (size_t(m) * gridDim.x + q) * tangents;
   for (int t = int(threadIdx.x); t < tangents; t += kBatchBlock) {
-    double c = 0.0;
-    if (q < nb_levels - 1 && t <= q) {
-      const double b = r0 + levels[t].altitude;
-      const double a1 = r0 + levels[q + 1].altitude, a0 = r0 + levels[q].altitude;
-      c = sqrt(a1 * a1 - b * b) - sqrt(a0 * a0 - b * b);
-    }
+    const double c = chordLength(levels, r0, nb_levels, q, t);
     if (chord) chord[row + t] = c;
     if (chord32) chord32[row + t] = float(c);
   }

@@ -340,6 +340,20 @@ __device__ __forceinline__ void waveTotals(double (&x)[K]) {
 // value of row r after waveTotals: 4b + kRowSlot[r]
 __device__ __forceinline__ int rowSlot(int row) { return row == 1 ? 2 : row == 2 ? 1 : row; }
 
+// Chord length of segment q on tangent path t (transmission_spectrum.cpp:
+// 117-118, 145-154): sqrt((R+z_{q+1})^2 - (R+z_t)^2) - sqrt((R+z_q)^2 -
+// (R+z_t)^2) for q >= t, zero for q < t and in the padding.  Evaluated
+// without contraction: fused, a*a - b*b at a == b leaves the rounding error
+// of b*b, which can be negative.
+__device__ __forceinline__ double chordLength(const LevelState* __restrict__ levels, double r0, int nb_levels, int q,
+                                              int t) {
+#pragma clang fp contract(off)
+  if (q >= nb_levels - 1 || t > q) return 0.0;
+  const double b = r0 + levels[t].altitude;
+  const double a1 = r0 + levels[q + 1].altitude, a0 = r0 + levels[q].altitude;
+  return sqrt(a1 * a1 - b * b) - sqrt(a0 * a0 - b * b);
+}
+
 // Optical depths of the tangent paths t0 .. t0+7 at this lane's wavenumber
 // (transmission_spectrum.cpp:107-139): tau_t = sum over q >= t of
 // c[t][q] (k_q + k_{q+1}) in increasing q, stopping at the first partial sum

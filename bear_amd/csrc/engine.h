@@ -336,7 +336,6 @@ class DeviceEngine {
   size_t speciesStride() const { return species_stride_; }
   size_t tableStride() const { return stride_; }          // elements per table row, a multiple of 64
   double* shifts() { return shift_host_; }
-  double* pathLengths() { return path_host_; }              // chord[segment][tangent] (transmission)
 
   // One evaluation: the high-resolution spectrum on the grid (kept on the
   // device; also written to spectrum_dev when given), the bins (also to
@@ -348,8 +347,10 @@ class DeviceEngine {
   void evaluateEmission(double scaling, double error_inflation, double* spectrum_dev, double* const* bins_dev);
   void evaluateEclipse(double star_temperature, double radius_ratio, double error_inflation, double* spectrum_dev,
                        double* const* bins_dev);
+  // isothermal: the staged levels are the model's own profile, not a given
+  // structure (setIsothermalStencils then holds for them)
   void evaluateTransmission(double bottom_radius, double star_radius, double error_inflation, double* spectrum_dev,
-                            double* const* bins_dev);
+                            double* const* bins_dev, bool isothermal);
   // eclipse depth against the tabulated stellar flux of uploadStellarSpectrum
   // (no bins): spectrum_dev = F / F_star (Rp/Rs)^2 1e6
   void evaluateEclipseTabulatedStar(double radius_ratio, double* spectrum_dev);
@@ -498,7 +499,6 @@ class DeviceEngine {
   LevelState* levels_host_ = nullptr;
   LevelSpecies* species_host_ = nullptr;
   double* shift_host_ = nullptr;
-  double* path_host_ = nullptr;
   double* ll_host_ = nullptr;
   double* ll_host_dev_ = nullptr;                // ll_host_ as the device addresses it
   // measurement

@@ -54,8 +54,8 @@ constexpr int kSplitBlock = 512;
 // chordSegments) and the partial effective heights [kTransmissionBlock /
 // tile][tile], FP64
 constexpr int kTransmissionBlock = 512;
-size_t transmissionLds(size_t nb_levels, size_t tile) {
-  return (size_t(chordSegments(int(nb_levels))) + kTransmissionBlock / tile) * tile * sizeof(double);
+size_t transmissionLds(size_t nb_levels, size_t tile, size_t threads = kTransmissionBlock) {
+  return (size_t(chordSegments(int(nb_levels))) + threads / tile) * tile * sizeof(double);
 }
 
 // Emission spectrum epilogue: the flux is kept for the bins; the optional
@@ -173,11 +173,11 @@ __global__ __launch_bounds__(kSplit ? kSplitBlock : kBlock) void emissionKernel(
 //     reference's trapezoid (one-sided at t = 0; T = 1 at the top level);
 //  3. per wavenumber, the partials in a fixed order, h = sqrt(H + R^2) - R and
 //     the depth (R_p + h)^2 / R_*^2 1e6 in FP64.
-// The transposed chord matrix chord[q][t] comes from the host.  EX: the H-
-// continuum joins the absorption and the clouds' layer optical depths join
+// The transposed chord matrix chord[q][t] comes from chordPointKernel.  EX: the
+// H- continuum joins the absorption and the clouds' layer optical depths join
 // as level extinction (transmission_spectrum.cpp:121-130).
-template <int NS, bool EX>
-__global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
+template <class Op, int kThreads, bool EX>
+__global__ __launch_bounds__(kThreads) void transmissionKernel(
     const double* __restrict__ tables, size_t stride, const double* __restrict__ rayleigh,
     const double* __restrict__ wavelength, Extras ex,
     const LevelState* __restrict__ levels, const LevelSpecies* __restrict__ species, StencilGroups stencil_groups,
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
   const int segments = chordSegments(L), tangents = chordTangents(L);
   double* S = lds;
   double* part = lds + size_t(segments) * tile;             // also the group-boundary levels of step 1
-  const int groups = kTransmissionBlock / tile;
+  const int groups = kThreads / tile;
   const int j = threadIdx.x % tile;
   const int g = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / tile);   // tile: a multiple of 64
   const int i = blockIdx.x * tile + j;
@@ -203,13 +203,13 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
   const int l1 = min(L, l0 + chunk);
   double last = 0.0;
   if (i < n) {
-    Opacity64<NS, false> op;
+    Op op;
     op.init(tables, nullptr, stride, i, exp_copy);
     const double sigma_r = rayleigh ? rayleigh[i] : 0.0;
     double hm[7], cf[kMaxClouds];
     if (EX) loadExtras(ex, i, n, wavelength[i], hm, cf);
     for (int l = l0; l < l1; ++l) {
-      const LevelSpecies* d = species + size_t(l) * NS;
+      const LevelSpecies* d = species + size_t(l) * Op::kNS;
       if (l == l0 || levels[l].reload != 0) op.load(d, levels[l], stencil_groups);
       double k = op.form(d, levels[l], stencil_groups) + sigma_r * levels[l].rayleigh_density;
       if (EX) {
@@ -257,6 +257,13 @@ __global__ __launch_bounds__(kTransmissionBlock) void transmissionKernel(
     depth[i] = d;
     if (spectrum) spectrum[i] = d;
   }
+}
+
+__global__ __launch_bounds__(kBlock) void chordPointKernel(const LevelState* __restrict__ levels, double bottom_radius,
+                                                           int nb_levels, double* __restrict__ chord) {
+  const int tangents = chordTangents(nb_levels);
+  for (int t = int(threadIdx.x); t < tangents; t += kBlock)
+    chord[size_t(blockIdx.x) * tangents + t] = chordLength(levels, bottom_radius, nb_levels, int(blockIdx.x), t);
 }
 
 // One workgroup per piece of a bin's segment (binChunkBody).
@@ -659,16 +666,15 @@ void DeviceEngine::configure(size_t nb_levels, size_t nb_species, bool transmiss
   if (staging_host_) (void)hipHostFree(staging_host_);
   deviceFree(staging_dev_);
   void* h = nullptr;
-  check(hipHostMalloc(&h, staging_bytes_ + sizeof(double), hipHostMallocDefault), "pinned staging");
+  check(hipHostMalloc(&h, off_path_ + sizeof(double), hipHostMallocDefault), "pinned staging");
   staging_host_ = static_cast<unsigned char*>(h);
-  std::memset(staging_host_, 0, staging_bytes_ + sizeof(double));
+  std::memset(staging_host_, 0, off_path_ + sizeof(double));
   staging_dev_ = deviceAlloc<unsigned char>(staging_bytes_, "per-evaluation inputs");
   levels_host_ = reinterpret_cast<LevelState*>(staging_host_);
   species_host_ = reinterpret_cast<LevelSpecies*>(staging_host_ + off_species_);
   for (size_t s = 0; s < species_stride_; ++s) species_host_[s].reload = 1;   // level 0 always loads
   shift_host_ = reinterpret_cast<double*>(staging_host_ + off_shift_);
-  path_host_ = transmission ? reinterpret_cast<double*>(staging_host_ + off_path_) : nullptr;
-  ll_host_ = reinterpret_cast<double*>(staging_host_ + staging_bytes_);
+  ll_host_ = reinterpret_cast<double*>(staging_host_ + off_path_);
   void* mapped = nullptr;
   check(hipHostGetDevicePointer(&mapped, ll_host_, 0), "hipHostGetDevicePointer");
   ll_host_dev_ = static_cast<double*>(mapped);
@@ -676,7 +682,7 @@ void DeviceEngine::configure(size_t nb_levels, size_t nb_species, bool transmiss
 
 void DeviceEngine::upload() {
   check(hipSetDevice(device_), "hipSetDevice");
-  check(hipMemcpyAsync(buffers().staging, staging_host_, staging_bytes_, hipMemcpyHostToDevice,
+  check(hipMemcpyAsync(buffers().staging, staging_host_, off_path_, hipMemcpyHostToDevice,
                        static_cast<hipStream_t>(stream_)),
         "upload inputs");
 }
@@ -864,7 +870,7 @@ void DeviceEngine::copyFlux(double* host) {
 }
 
 void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius, double inflation,
-                                        double* spectrum_dev, double* const* bins_dev) {
+                                        double* spectrum_dev, double* const* bins_dev, bool isothermal) {
   if (!transmission_) raise(kInvalidInput, "the engine is not configured for transmission");
   requireFP64Tables("the single-model path");
   upload();
@@ -872,30 +878,39 @@ void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius
   hipStream_t s = static_cast<hipStream_t>(stream_);
   const LevelState* lev = reinterpret_cast<const LevelState*>(buf.staging);
   const LevelSpecies* spc = reinterpret_cast<const LevelSpecies*>(buf.staging + off_species_);
-  const double* path = reinterpret_cast<const double*>(buf.staging + off_path_);
+  double* path = reinterpret_cast<double*>(buf.staging + off_path_);
   const int n = int(n_points_), L = int(nb_levels_);
+  const Extras ex = extras();
+  hipLaunchKernelGGL(chordPointKernel, dim3(unsigned(chordSegments(L))), dim3(kBlock), 0, s, lev, bottom_radius, L,
+                     path);
+  check(hipGetLastError(), "chord kernel");
+  beginTimed();
   // tiles of 128 or 64 wavenumbers, the wider one when its LDS (the segment
   // sums and the partials) fits the workgroup
-  const int tile = transmissionLds(L, 128) <= lds_limit_ ? 128 : 64;
-  size_t lds = transmissionLds(L, tile);
-  int exp_offset = 0;
-  if (lds + kExpTable * sizeof(double) <= lds_limit_) {
-    exp_offset = int(lds / sizeof(double));
-    lds += kExpTable * sizeof(double);
-  }
-  const int blocks = (n + tile - 1) / tile;
-  const Extras ex = extras();
-  beginTimed();
+  auto launch = [&](auto op, auto threads, auto extra) {
+    const int tile = transmissionLds(L, 128, threads) <= lds_limit_ ? 128 : 64;
+    size_t lds = transmissionLds(L, tile, threads);
+    int exp_offset = 0;
+    if (lds + kExpTable * sizeof(double) <= lds_limit_) {
+      exp_offset = int(lds / sizeof(double));
+      lds += kExpTable * sizeof(double);
+    }
+    hipLaunchKernelGGL((transmissionKernel<decltype(op), decltype(threads)::value, decltype(extra)::value>), dim3(unsigned((n + tile - 1) / tile)),
+                       dim3(threads), lds, s, tables_, stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path,
+                       L, n, tile, bottom_radius, star_radius, buf.flux, spectrum_dev, exp_offset);
+  };
   const bool launched = withSlots(species_stride_, [&](auto ns) {
     constexpr int NS = ns;
-    if (hasExtras(ex))
-      hipLaunchKernelGGL((transmissionKernel<NS, true>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
-                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
-                         star_radius, buf.flux, spectrum_dev, exp_offset);
-    else
-      hipLaunchKernelGGL((transmissionKernel<NS, false>), dim3(blocks), dim3(kTransmissionBlock), lds, s, tables_,
-                         stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n, tile, bottom_radius,
-                         star_radius, buf.flux, spectrum_dev, exp_offset);
+    // the isothermal stencils and their wavefronts as in the batched kernel
+    // (120 levels, 7 slots, 60,013 wavenumbers, with the chords formed here
+    // instead of on the host: 249 -> 178 us per call)
+    constexpr int kWide = NS <= 12 ? 1024 : 512;
+    using Wide = std::integral_constant<int, kWide>;
+    using Block = std::integral_constant<int, kTransmissionBlock>;
+    if (hasExtras(ex)) launch(Opacity64<NS, false>{}, Block{}, std::true_type{});
+    else if (isothermal && isothermal_ && transmissionLds(L, 64, kWide) + kExpTable * sizeof(double) <= lds_limit_)
+      launch(Opacity64Isothermal<NS>{}, Wide{}, std::false_type{});
+    else launch(Opacity64<NS, false>{}, Block{}, std::false_type{});
   });
   if (!launched) raise(kInvalidInput, "unsupported number of species for transmission");
   check(hipGetLastError(), "transmission kernel");

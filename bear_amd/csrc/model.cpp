@@ -869,34 +869,12 @@ void TransmissionModel::gradientBatch(const double* params, size_t batch, size_t
   if (!failure.empty()) raise(failure_code, failure);
 }
 
-// chord lengths between successive levels for every tangent level
-// (transmission_spectrum.cpp:117-118, 145-154), transposed: chord[i][t] =
-// sqrt((R+z_{i+1})^2 - (R+z_t)^2) - sqrt((R+z_i)^2 - (R+z_t)^2), i >= t
-// (the entries with i < t and the padding stay zero)
-void TransmissionModel::stageChords(double r0) {
-  const size_t L = atmosphere_.nb_levels;
-  const size_t tangents = size_t(chordTangents(int(L)));
-  const std::vector<double>& z = atmosphere_.altitude;
-  double* chord = engine_.pathLengths();
-  for (size_t t = 0; t + 1 < L; ++t) {
-    const double b = r0 + z[t];
-    double previous = std::sqrt(b * b - b * b);
-    for (size_t i = t; i + 1 < L; ++i) {
-      const double a = r0 + z[i + 1];
-      const double next = std::sqrt(a * a - b * b);
-      chord[i * tangents + t] = next - previous;
-      previous = next;
-    }
-  }
-}
-
 // TransmissionModel::calcModelGPU (transmission.cpp:257-321)
 bool TransmissionModel::calcModelGPU(const double* p, double inflation, double* spectrum_dev,
                                      double* const* spectrum_obs_dev) {
   BatchModel scalars;
   const bool neglect = stage(p, scalars);
-  stageChords(p[1]);
-  engine_.evaluateTransmission(p[1], p[2], inflation, spectrum_dev, spectrum_obs_dev);
+  engine_.evaluateTransmission(p[1], p[2], inflation, spectrum_dev, spectrum_obs_dev, true);
   return neglect;
 }
 
@@ -904,9 +882,9 @@ void TransmissionModel::calcSpectrum(double g, double planet_radius, double radi
                                      const double* t, const std::vector<int>& species, const double* x,
                                      bool variable_gravity, double* spectrum) {
   stageStructure(g, planet_radius, variable_gravity, p, t, species, x);
-  stageChords(planet_radius);
   double* dev = engine_.spectrumBuffer();
-  engine_.evaluateTransmission(planet_radius, planet_radius / radius_ratio, 0.0, dev, nullptr);   // transmission.cpp:391-392
+  engine_.evaluateTransmission(planet_radius, planet_radius / radius_ratio, 0.0, dev, nullptr,
+                               false);                           // transmission.cpp:391-392
   engine_.copySpectrum(spectrum, dev);
 }
 

@@ -238,8 +238,6 @@ class TransmissionModel : public TabulatedModel {
   double fixedScaleHeight(const double* p) const override { return fit_scale_height_ ? p[3] : 0.0; }
   int altitudeKind() const override { return fit_mmw_ ? 1 : fit_scale_height_ ? 2 : 0; }
   bool variableGravity() const override { return variable_gravity_; }
-  // the chord lengths of the staged atmosphere into the engine's staging
-  void stageChords(double bottom_radius);
   bool fit_mmw_ = false, fit_scale_height_ = false, variable_gravity_ = false;
 };
 
