@@ -397,17 +397,23 @@ __device__ __forceinline__ void tangentBlock(const K* __restrict__ seg, int tile
     for (int k = 0; k < kTangentBlock; ++k) {
       const bool past = tau[k] > K(10);
       const bool first = past && fin[k] == K(0);
-      if (__builtin_amdgcn_ballot_w64(first) != 0) {       // uniform branch: exact re-sum of path k
-        K x = prev[k], hit = K(0);
-        int hit_q = 0;
-        bool found = false;
+      // uniform branch: exact re-sum of path k, told unlikely so that it stays
+      // a branch (executed for every path, 100 transits of 100 levels on INT16
+      // tables take 4.96 ms instead of 3.87) out of the way of the others
+      if (__builtin_expect_with_probability(__builtin_amdgcn_ballot_w64(first) != 0, 0, 0.999)) {
+        // the sums after each segment of the step; the first one above 10
+        // counts (tau[k], after the last, is), so the earlier override
+        K x[kSegmentStep];
+        x[0] = fma(c[k], sq[0], prev[k]);
 #pragma unroll
-        for (int u = 0; u < kSegmentStep; ++u) {
-          x = fma(c[u * tangents + k], sq[u], x);
-          const bool now = !found && x > K(10);
-          hit = now ? x : hit;
-          if constexpr (kStop) hit_q = now ? q0 + u : hit_q;
-          found = found || now;
+        for (int u = 1; u < kSegmentStep - 1; ++u) x[u] = fma(c[u * tangents + k], sq[u], x[u - 1]);
+        K hit = tau[k];
+        int hit_q = q0 + kSegmentStep - 1;
+#pragma unroll
+        for (int u = kSegmentStep - 2; u >= 0; --u) {
+          const bool above = x[u] > K(10);
+          hit = above ? x[u] : hit;
+          if constexpr (kStop) hit_q = above ? q0 + u : hit_q;
         }
         fin[k] = first ? hit : fin[k];
         if constexpr (kStop) last[k] = first ? hit_q : last[k];
