@@ -1,11 +1,12 @@
 // Batched likelihood evaluation on gfx950: many live points of one retrieval
 // per launch sequence.
 //
-// One work item is (wavenumber tile, live point).  The spectrum kernels are
-// persistent: a grid sized by the autotuner walks the items, ordered so that
-// every live point of one tile runs on the same XCD (workgroups go to XCDs
-// round-robin by id, and the grid is a multiple of 8), where the tile's
-// table rows stay in that XCD's L2 while the points reuse them.
+// One work item is (wavenumber tile, live point), ordered so that every live
+// point of one tile runs on the same XCD (workgroups go to XCDs round-robin by
+// id, and the grid is a multiple of 8), where the tile's table rows stay in
+// that XCD's L2 while the points reuse them.  A workgroup takes one item, and
+// the dispatcher levels them; only the FP64 transits walk the items with a
+// persistent grid, sized by the autotuner.
 //
 // Per batch, in one hipGraph when enabled: the pinned per-point records go to
 // the device in one copy; (transmission) the chord lengths of every point are

@@ -308,7 +308,7 @@ typedef struct bear_batch_stats {
   int precision;                 /* BEAR_TABLE_* */
   int block;                     /* launch shape of the last batch: threads per workgroup */
   int tile;                      /* wavenumbers per work item */
-  int grid;                      /* persistent workgroups */
+  int grid;                      /* workgroups */
   int used_graph;
   size_t evaluations;            /* live points evaluated in batches */
   double gpu_ms_total;           /* device time of those batches (with profiling on) */
