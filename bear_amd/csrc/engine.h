@@ -262,7 +262,7 @@ struct StagePlan {
 struct BatchLaunch {
   int block = 256;               // threads per workgroup
   int tile = 256;                // wavenumbers per work item
-  int grid = 0;                  // workgroups (transmission: persistent)
+  int grid = 0;                  // workgroups (FP64 transits: persistent; else one per item)
   int group = 32;                // points per group of the work-item order (transmission)
   int split = 1;                 // emission: wavefronts that share one tile's levels
 };

@@ -10,8 +10,8 @@
 //   weights                  folded observation operator, one contiguous
 //                            segment per bin
 //   bins, ll_terms           [bins] FP64
-// Per evaluation the host fills one pinned block (levels, stencils, shifts,
-// chord lengths) that is copied in one transfer.
+// Per evaluation the host fills one pinned block (levels, stencils, shifts)
+// that is copied in one transfer.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
