@@ -23,6 +23,7 @@
 #include "device_math.h"
 #include "emission_sweep.h"
 #include "engine.h"
+#include "launch_shape.h"
 
 namespace bear_amd {
 
@@ -49,14 +50,7 @@ void check(hipError_t e, const char* what) {
 constexpr int kBlock = 128;
 // Few tiles: workgroups of 4 or 8 wavefronts share one tile's levels
 constexpr int kSplitBlock = 512;
-// Single-point transmission: workgroups of 8 wavefronts share one tile's
-// segment extinction sums in LDS (S[segment][tile], rows padded to
-// chordSegments) and the partial effective heights [kTransmissionBlock /
-// tile][tile], FP64
-constexpr int kTransmissionBlock = 512;
-size_t transmissionLds(size_t nb_levels, size_t tile, size_t threads = kTransmissionBlock) {
-  return (size_t(chordSegments(int(nb_levels))) + threads / tile) * tile * sizeof(double);
-}
+static_assert(kExpTableBytes == kExpTable * sizeof(double), "transit shapes laid out for another table");
 
 // Emission spectrum epilogue: the flux is kept for the bins; the optional
 // high-resolution output is F per micron (radiative_transfer.h:58-60) for
@@ -652,7 +646,7 @@ void DeviceEngine::configure(size_t nb_levels, size_t nb_species, bool transmiss
   species_stride_ = stencilSlots(nb_species);                        // padding entries keep n = 0, row 0
   if (transmission && species_stride_ > kMaxSlots)
     raise(kInvalidInput, "the transmission model takes at most 16 tabulated species");
-  if (transmission && transmissionLds(nb_levels, 64) > lds_limit_)
+  if (transmission && transitLds(int(nb_levels), 64, kTransitThreads) > lds_limit_)
     raise(kInvalidInput, "too many levels for the transmission kernel");
   const size_t lv = (nb_levels * sizeof(LevelState) + 63) / 64 * 64;      // stencil records start 64-B aligned
   const size_t sp = nb_levels * species_stride_ * sizeof(LevelSpecies);
@@ -885,32 +879,21 @@ void DeviceEngine::evaluateTransmission(double bottom_radius, double star_radius
                      path);
   check(hipGetLastError(), "chord kernel");
   beginTimed();
-  // tiles of 128 or 64 wavenumbers, the wider one when its LDS (the segment
-  // sums and the partials) fits the workgroup
-  auto launch = [&](auto op, auto threads, auto extra) {
-    const int tile = transmissionLds(L, 128, threads) <= lds_limit_ ? 128 : 64;
-    size_t lds = transmissionLds(L, tile, threads);
-    int exp_offset = 0;
-    if (lds + kExpTable * sizeof(double) <= lds_limit_) {
-      exp_offset = int(lds / sizeof(double));
-      lds += kExpTable * sizeof(double);
-    }
-    hipLaunchKernelGGL((transmissionKernel<decltype(op), decltype(threads)::value, decltype(extra)::value>), dim3(unsigned((n + tile - 1) / tile)),
-                       dim3(threads), lds, s, tables_, stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path,
-                       L, n, tile, bottom_radius, star_radius, buf.flux, spectrum_dev, exp_offset);
+  // the isothermal stencils and their wavefronts as in the batched kernel (120
+  // levels, 7 slots, 60,013 wavenumbers, with the chords formed here instead
+  // of on the host: 249 -> 178 us per call)
+  const bool extra = hasExtras(ex);
+  const TransitShape shape = transitShape(L, species_stride_, isothermal && isothermal_ && !extra, lds_limit_);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned((n + shape.tile - 1) / shape.tile)), dim3(unsigned(shape.threads)),
+                       shape.lds, s, tables_, stride_, rayleigh_, wavelength_, ex, lev, spc, groups_, path, L, n,
+                       shape.tile, bottom_radius, star_radius, buf.flux, spectrum_dev, shape.exp_offset);
   };
   const bool launched = withSlots(species_stride_, [&](auto ns) {
     constexpr int NS = ns;
-    // the isothermal stencils and their wavefronts as in the batched kernel
-    // (120 levels, 7 slots, 60,013 wavenumbers, with the chords formed here
-    // instead of on the host: 249 -> 178 us per call)
-    constexpr int kWide = NS <= 12 ? 1024 : 512;
-    using Wide = std::integral_constant<int, kWide>;
-    using Block = std::integral_constant<int, kTransmissionBlock>;
-    if (hasExtras(ex)) launch(Opacity64<NS, false>{}, Block{}, std::true_type{});
-    else if (isothermal && isothermal_ && transmissionLds(L, 64, kWide) + kExpTable * sizeof(double) <= lds_limit_)
-      launch(Opacity64Isothermal<NS>{}, Wide{}, std::false_type{});
-    else launch(Opacity64<NS, false>{}, Block{}, std::false_type{});
+    if (extra) launch(transmissionKernel<Opacity64<NS, false>, kTransitThreads, true>);
+    else if (shape.isothermal) launch(transmissionKernel<Opacity64Isothermal<NS>, isothermalThreads(NS), false>);
+    else launch(transmissionKernel<Opacity64<NS, false>, kTransitThreads, false>);
   });
   if (!launched) raise(kInvalidInput, "unsupported number of species for transmission");
   check(hipGetLastError(), "transmission kernel");

@@ -1,0 +1,58 @@
+// Launch shapes that follow from sizes alone, apart from the kernels, so that
+// every size can be checked without a device.
+#pragma once
+
+#include <cstddef>
+
+#include "engine.h"
+
+namespace bear_amd {
+
+// LDS of a transit workgroup: the segment extinction sums of its tile
+// (S[segment][tile], rows padded to chordSegments) and the partial effective
+// heights [threads / tile][tile], FP64
+constexpr size_t transitLds(int levels, int tile, int threads) {
+  return (size_t(chordSegments(levels)) + size_t(threads / tile)) * size_t(tile) * sizeof(double);
+}
+
+// the exponential table in LDS (exp_table.h)
+constexpr size_t kExpTableBytes = 128 * 16 * sizeof(double);
+
+// Threads of a workgroup over general stencils: 8 wavefronts share one tile;
+// over isothermal ones 16 up to 12 slots (128 registers: beyond that the
+// slots' values spill), 8 above.
+constexpr int kTransitThreads = 512;
+constexpr int isothermalThreads(size_t slots) { return slots <= 12 ? 1024 : kTransitThreads; }
+
+// The single-point transit kernel's form and shape for `levels` levels and
+// `slots` stencil slots, within `lds_limit` bytes of LDS.
+struct TransitShape {
+  bool isothermal;               // two-value stencils: they have no other exponential than the table's
+  int threads, tile;             // tile: wavenumbers per workgroup
+  int exp_offset;                // of the exponential table in the LDS doubles; 0: no room, no table
+  size_t lds;                    // bytes
+};
+
+// Isothermal stencils where the model has them and the table fits beside the
+// sums of the tile that is launched: tiles of 128 wavenumbers, else of 64;
+// otherwise the general stencils, on the wider tile that fits and with the
+// table only where there is room beside it.  One transit of 7 slots and 46,935
+// wavenumbers, general -> isothermal, per likelihood: 136 levels (tile 128)
+// 252 -> 149 us, 150 levels (tile 64) 286 -> 157 us, 200 levels 342 -> 201 us.
+constexpr TransitShape transitShape(int levels, size_t slots, bool isothermal, size_t lds_limit) {
+  if (isothermal) {
+    const int threads = isothermalThreads(slots);
+    for (int tile : {128, 64}) {
+      const size_t sums = transitLds(levels, tile, threads);
+      if (sums + kExpTableBytes <= lds_limit)
+        return {true, threads, tile, int(sums / sizeof(double)), sums + kExpTableBytes};
+    }
+  }
+  const int tile = transitLds(levels, 128, kTransitThreads) <= lds_limit ? 128 : 64;
+  const size_t sums = transitLds(levels, tile, kTransitThreads);
+  if (sums + kExpTableBytes <= lds_limit)
+    return {false, kTransitThreads, tile, int(sums / sizeof(double)), sums + kExpTableBytes};
+  return {false, kTransitThreads, tile, 0, sums};
+}
+
+}  // namespace bear_amd

@@ -64,7 +64,8 @@ struct Opacity64 {
 // loaded, and a slot keeps its value at the lower pressure row and the step
 // to the upper one, in the table's units.  Half the registers, which lets 16
 // wavefronts share a tile of 200 levels where 8 could, and two operations per
-// slot and level fewer.
+// slot and level fewer.  The launch has to bring the table (exp_copy not
+// null): transitShape and launchTransmission take this form only where it fits.
 template <int NS>
 struct Opacity64Isothermal {
   static constexpr int kNS = NS;

@@ -1,0 +1,58 @@
+"""Launch shapes for every size, on the host: bear_amd/csrc/launch_shape.h
+compiled by the host compiler."""
+
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+CSRC = os.path.join(ROOT, "bear_amd", "csrc")
+LDS = 160 * 1024                                        # per workgroup on gfx950
+TABLE = 16 * 1024                                       # the exponential table
+
+
+def _run(folder, body):
+    src = os.path.join(folder, "shapes.cpp")
+    with open(src, "w") as f:
+        f.write('#include <cstdio>\n#include "launch_shape.h"\nusing namespace bear_amd;\nint main() {\n' + body + "}\n")
+    exe = os.path.join(folder, "shapes")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, "-I", os.path.join(ROOT, "include"), src, "-o", exe],
+                   check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+    return [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+
+
+@pytest.mark.parametrize("limit", [64 * 1024, LDS])
+def test_single_transit_shapes(tmp_path, limit):
+    """Two-value stencils never without their table, and every form within the
+    workgroup's LDS, the table behind the sums of the tile that is launched."""
+    rows = _run(str(tmp_path), """
+  for (int L = 2; L <= 400; ++L)
+    for (int slots = 1; slots <= 16; ++slots)
+      for (int iso = 0; iso < 2; ++iso) {
+        if (transitLds(L, 64, kTransitThreads) > %d) continue;      // refused when the model is configured
+        const TransitShape s = transitShape(L, slots, iso, %d);
+        std::printf("%%d %%d %%d %%d %%d %%d %%d %%zu %%d\\n", L, slots, iso, int(s.isothermal), s.threads, s.tile,
+                    s.exp_offset, s.lds, chordSegments(L));
+      }
+""" % (limit, limit))
+    assert rows
+    forms = set()
+    for levels, slots, iso, isothermal, threads, tile, offset, lds, segments in rows:
+        sums = (segments + threads // tile) * tile * 8
+        assert tile in (64, 128) and threads % tile == 0 and segments >= levels - 1
+        assert lds <= limit
+        if isothermal:
+            assert iso and offset * 8 == sums and lds == sums + TABLE
+            assert threads == (1024 if slots <= 12 else 512)
+        else:
+            assert threads == 512
+            assert (offset * 8 == sums and lds == sums + TABLE) or (offset == 0 and lds == sums)
+            if iso:                                          # given up only where no tile leaves room for the table
+                wide = 1024 if slots <= 12 else 512
+                assert (segments + wide // 64) * 64 * 8 + TABLE > limit
+        forms.add((isothermal, tile, offset > 0))
+    if limit == LDS:
+        assert forms == {(1, 128, True), (1, 64, True), (0, 128, True), (0, 128, False), (0, 64, True), (0, 64, False)}
