@@ -165,11 +165,12 @@ size_t transmissionBatchLds(int L, int tile, bool wide, int threads) {
 
 // ---------------------------------------------------------------- precision
 // residual tables [rows][stride] and the base [slots][stride], zero base in
-// the padding slots (their density is zero)
+// the padding slots (their density is zero, their row is row 0)
 void DeviceEngine::allocateReduced(TablePrecision p, size_t nb_rows, size_t slots) {
   void* low = nullptr;
-  check(hipMalloc(&low, std::max<size_t>(1, nb_rows) * stride_ * tableElementBytes(p)), "reduced-precision tables");
+  check(hipMalloc(&low, nb_rows * stride_ * tableElementBytes(p)), "reduced-precision tables");
   tables_low_ = low;
+  check(hipMemsetAsync(low, 0, stride_ * tableElementBytes(p), static_cast<hipStream_t>(stream_)), "clear table row");
   base_rows_ = slots * (p == TablePrecision::int16 ? 2 : 1);          // int16: base and scale per slot
   table_base_ = deviceAlloc<float>(base_rows_ * stride_, "table base");
   check(hipMemsetAsync(table_base_, 0, base_rows_ * stride_ * sizeof(float), static_cast<hipStream_t>(stream_)),

@@ -478,14 +478,17 @@ void DeviceEngine::allocateTables(size_t nb_rows, size_t nb_species) {
     raise(kInvalidInput, "tables too large: rows x wavenumbers exceeds 2^38 values");
   deviceFree(tables_);
   tables_ = nullptr;
-  n_rows_ = nb_rows;
+  // padding slots read row 0, so there is one also without tabulated species
+  // (only the H- continuum or a Rayleigh scatterer listed), of zeros then
+  n_rows_ = std::max<size_t>(1, nb_rows);
   if (storage_ == TablePrecision::fp64) {
-    tables_ = deviceAlloc<double>(nb_rows * stride_, "cross-section tables");
+    tables_ = deviceAlloc<double>(n_rows_ * stride_, "cross-section tables");
+    check(hipMemsetAsync(tables_, 0, stride_ * sizeof(double), static_cast<hipStream_t>(stream_)), "clear table row");
     return;
   }
   // residual rows and the per-species base only; every species passes
   // through an FP64 staging buffer of its own rows (uploadSpeciesRows)
-  allocateReduced(storage_, nb_rows, stencilSlots(nb_species));
+  allocateReduced(storage_, n_rows_, stencilSlots(nb_species));
 }
 
 void DeviceEngine::uploadSpeciesRows(int slot, size_t first, size_t count, const double* rows) {
