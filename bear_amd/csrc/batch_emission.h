@@ -97,7 +97,7 @@ __global__ __launch_bounds__((kBatchBlock), (sweepWaves<Op, EX>())) void emissio
   }
   op.load(species, levels[0], rec.groups);
   double k_prev = op.form(species, levels[0], rec.groups);
-  if (EX && e.hminus) k_prev += hminusKappa(hm, levels[0]);
+  if (EX && e.hminus) k_prev = withHminus(k_prev, hm, levels[0]);
   double b_prev = col.planck(levels[0]), d1 = 0.0, d2 = 0.0;       // I = B at the bottom
   float* kept = keep + keptColumn(m, stride, nb_levels, i);
   if (keep) {
@@ -109,7 +109,7 @@ __global__ __launch_bounds__((kBatchBlock), (sweepWaves<Op, EX>())) void emissio
     const Species* d = species + size_t(l) * Op::kNS;
     if (levels[l].reload) op.load(d, levels[l], rec.groups);
     double k_next = op.form(d, levels[l], rec.groups);
-    if (EX && e.hminus) k_next += hminusKappa(hm, levels[l]);
+    if (EX && e.hminus) k_next = withHminus(k_next, hm, levels[l]);
     const double b_next = col.planck(levels[l]);
     double tau = levels[l].half_dz * (k_next + k_prev);
     if (EX) tau += cloudLayer(e, cf, levels[l], l, i, n);

@@ -212,6 +212,15 @@ __device__ __forceinline__ double hminusKappa(const double (&hm)[7], const Level
   return k;
 }
 
+// A level's emission opacity with the H- continuum joined to the tabulated
+// kappa k.  Where the level holds no tabulated absorber, k (a zero density is
+// 2^-340 in the table's exponentials) counts as an exact 0: H- rows are 0 at
+// some wavelengths, and a layer of optical depth 0 passes the intensity on
+// unchanged, one of any other does not.
+__device__ __forceinline__ double withHminus(double k, const double (&hm)[7], const LevelState& lev) {
+  return hminusKappa(hm, lev) + (lev.absorbers != 0 ? k : 0.0);
+}
+
 // per thread, once: the H- rows and the cloud models' spectral factors at
 // wavelength lam (micron) (power_law_cloud_model.cpp:114-120,
 // kh_cloud_model.cpp:116-132); unused slots are zero

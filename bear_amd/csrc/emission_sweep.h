@@ -112,9 +112,8 @@ __device__ __forceinline__ double sweepDown(Op& op, const typename Op::Species* 
   const int ns = op.slots();
   auto level = [&](int l) { return species + size_t(l) * ns; };
   auto form = [&](int l) {
-    double k = double(op.form(level(l), levels[l], groups));
-    if (EX && e.hminus) k += hminusKappa(hm, levels[l]);
-    return k;
+    const double k = double(op.form(level(l), levels[l], groups));
+    return EX && e.hminus ? withHminus(k, hm, levels[l]) : k;
   };
   int l = runTop(nb_levels, first);
   op.load(level(l), levels[l], groups);

@@ -43,8 +43,9 @@ struct Extras {
 // first, in whole lines of the scalar cache.
 struct alignas(64) LevelState {
   double inv_temperature;
-  // half the thickness of the layer below this level; 0 at level 0, and where
-  // neither level holds a tabulated absorber (no opacity: an exact 0)
+  // half the thickness of the layer below this level; 0 at level 0, and, in a
+  // model without the H- continuum, where neither level holds a tabulated
+  // absorber (no opacity: an exact 0; with H-, withHminus sees to it)
   double half_dz;
   double altitude;
   double rayleigh_density;   // number density of the Rayleigh scatterer (transmission)

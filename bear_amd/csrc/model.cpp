@@ -221,7 +221,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       }
       lev[l].reload |= changed << s;
     }
-    if (l > 0 && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
+    if (l > 0 && !hminus_ && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
   }
   size_t k = 0;                                                   // forward_model.cpp:184-204
   for (size_t o = 0; o < observations_.size(); ++o) {
