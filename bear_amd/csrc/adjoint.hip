@@ -46,6 +46,7 @@
 #include <string>
 
 #include "device_math.h"
+#include "launch_shape.h"
 #include "tile_window.h"
 #include "engine.h"
 
@@ -1072,9 +1073,9 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
   const int tiles = (n + kWave - 1) / kWave;
   const int grid = int(align8(std::max<size_t>(8, size_t(nb_cus_) * kAdjointWavesPerCu)));
 
-  // points per chunk: kept forward quantities within the budget (and 80 % of
-  // the free memory, checked when the buffers grow), else recomputed
-  // (emission and eclipse); transmission also holds per point the chord
+  // points per chunk: what a launch takes, and kept forward quantities within
+  // the budget (and 80 % of the free memory, checked when the buffers grow),
+  // else recomputed (emission and eclipse); transmission also holds per point the chord
   // gradients and their per-range partial sums, and when one point's kept
   // quantities exceed the budget it takes one point at a time with its grid
   // in windows of whole chord ranges, running the forward kernel again with
@@ -1102,8 +1103,9 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
   size_t chunk = 0, buffer_size = 0, partial_size = 0;
   int window_ranges = ranges;                                                  // chord ranges per window
   bool kept = false;
+  const size_t launchable = std::min(batch, pointsPerLaunch(tiles, kWave));
   auto plan = [&] {
-    chunk = std::min(batch, budget / (kept_point * sizeof(double)));
+    chunk = std::min(launchable, budget / (kept_point * sizeof(double)));
     kept = chunk > 0;
     window_ranges = ranges;
     if (!kept && transmission) {
@@ -1116,7 +1118,7 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
       }
     }
     if (!kept)
-      chunk = std::min(batch, std::max<size_t>(1, kPartialBudget / ((partial_point + stride_) * sizeof(double))));
+      chunk = std::min(launchable, std::max<size_t>(1, kPartialBudget / ((partial_point + stride_) * sizeof(double))));
     const size_t chunks = (batch + chunk - 1) / chunk;                      // equal chunks, no small tail
     chunk = (batch + chunks - 1) / chunks;
     if (!kept) buffer_size = size_t(grid) * L * 2 * kWave;                   // doubles

@@ -25,6 +25,7 @@
 #include "batch_launch.h"
 #include "device_math.h"
 #include "engine.h"
+#include "launch_shape.h"
 #include "reduced_opacity.h"
 #include "tile_window.h"
 
@@ -345,7 +346,15 @@ void DeviceEngine::launchBatchSpectrum(ModelKind kind, size_t batch, const Batch
     }
     launched = launchTransmissionSlots1To8(species_stride_, a) || launchTransmissionSlots9To16(species_stride_, a);
   } else {
-    launched = launchEmissionSlots1To8(species_stride_, a) || launchEmissionSlots9To16(species_stride_, a);
+    const size_t run = pointsPerLaunch((n + lc.tile - 1) / lc.tile, lc.block);
+    launched = true;
+    for (size_t m = 0; m < batch && launched; m += run) {
+      a.batch = int(std::min(run, batch - m));
+      a.rec.base = rec.base + m * rec_bytes_;
+      a.flux = flux + m * stride_;
+      a.keep = keep ? keep + m * (stride_ / kKeptValue) * size_t(L) * kKeptLevel : nullptr;   // keptColumn
+      launched = launchEmissionSlots1To8(species_stride_, a) || launchEmissionSlots9To16(species_stride_, a);
+    }
   }
   if (!launched) raise(kInvalidInput, "the batched kernels take at most 16 tabulated species");
   check(hipGetLastError(), "batched spectrum kernel");

@@ -1,7 +1,10 @@
 // Batched transit spectra: the kernel and its launch by precision.
 #pragma once
 
+#include <algorithm>
+
 #include "batch_launch.h"
+#include "launch_shape.h"
 #include "opacity64.h"
 #include "reduced_opacity.h"
 
@@ -178,8 +181,10 @@ void launchTransmissionKernel(const SpectrumBatch& a, const void* tab) {
   }
   // FP64: a persistent grid, whose workgroups fill their exponential table
   // once; reduced precision: one item per workgroup, levelled by the
-  // dispatcher (100 transits of 100 levels on INT16 tables 4.4 -> 4.0 ms)
-  const unsigned grid = wide ? unsigned(a.shape.grid) : unsigned(nbItems(a.win.count, a.batch));
+  // dispatcher (100 transits of 100 levels on INT16 tables 4.4 -> 4.0 ms), as
+  // far as a launch goes
+  const unsigned grid = wide ? unsigned(a.shape.grid)
+                             : unsigned(std::min(nbItems(a.win.count, a.batch), maxWorkgroups(kThreads)));
   hipLaunchKernelGGL((transmissionBatchKernel<Op, kThreads, kKeep, EX>), dim3(grid), dim3(kThreads), lds,
                      a.stream, tab, a.base, a.stride, a.rayleigh, a.wavelength, a.ex, a.rec, a.chord, a.chord32,
                      a.levels, a.n, a.win, a.shape.tile, a.batch, a.shape.group, a.flux, a.keep, a.reach, exp_offset);
@@ -194,7 +199,7 @@ void launchTransmission(const SpectrumBatch& a) {
       // 12 slots (128 registers: beyond that the slots' values spill), 8 above.
       // 200 transits, 12 slots, 200 levels: 11.35 -> 8.96 ms against the
       // general stencils.  Both go through the same tangent sums, 4 ms of it.
-      constexpr int kWide = NS <= 12 ? 1024 : 512;
+      constexpr int kWide = isothermalThreads(NS);
       if (a.isothermal && !a.extras &&
           transmissionBatchLds(a.levels, a.shape.tile, true, kWide) + kExpTable * sizeof(double) <= a.lds_limit)
         return a.keep ? launchTransmissionKernel<Opacity64Isothermal<NS>, kWide, true, false>(a, a.tab64)

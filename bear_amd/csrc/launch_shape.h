@@ -55,4 +55,15 @@ constexpr TransitShape transitShape(int levels, size_t slots, bool isothermal, s
   return {false, kTransitThreads, tile, 0, sums};
 }
 
+// A launch takes fewer than 2^32 threads in x.  Workgroups at most, in whole
+// rounds of the 8 XCDs (device_math.h, workItem).
+constexpr size_t maxWorkgroups(int threads) { return ((size_t(1) << 32) - 1) / size_t(threads) / 8 * 8; }
+
+// Live points per launch of a kernel with one workgroup of `threads` per
+// (tile, point): larger batches take several launches.
+constexpr size_t pointsPerLaunch(int tiles, int threads) {
+  const size_t points = maxWorkgroups(threads) / (size_t((tiles + 7) / 8) * 8);
+  return points > 0 ? points : 1;
+}
+
 }  // namespace bear_amd

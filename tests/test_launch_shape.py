@@ -56,3 +56,27 @@ def test_single_transit_shapes(tmp_path, limit):
         forms.add((isothermal, tile, offset > 0))
     if limit == LDS:
         assert forms == {(1, 128, True), (1, 64, True), (0, 128, True), (0, 128, False), (0, 64, True), (0, 64, False)}
+
+
+def test_launches_of_large_batches(tmp_path):
+    """Every launch below 2^32 threads, at most 65,535 points per batch, and
+    no more launches than that takes."""
+    sizes = [1, 63, 64, 65, 2554, 16_500, 60_000, 65_600, 400_000, 1_000_003]
+    rows = _run(str(tmp_path), """
+  for (int n : {%s})
+    for (int tile : {64, 128, 256})
+      for (int threads : {64, 128, 256, 512})
+        std::printf("%%d %%d %%d %%zu %%zu\\n", n, tile, threads, pointsPerLaunch((n + tile - 1) / tile, threads),
+                    maxWorkgroups(threads));
+""" % ", ".join(str(n) for n in sizes))
+    assert len(rows) == len(sizes) * 12
+    split = 0
+    for n, tile, threads, points, groups in rows:
+        per_point = (-(-n // tile) + 7) // 8 * 8
+        assert points >= 1 and groups % 8 == 0 and groups * threads < 2 ** 32 <= (groups + 8) * threads
+        assert points * per_point <= groups < (points + 1) * per_point
+        for batch in (1, 8950, 10_737, 65_535):
+            runs = [min(points, batch - m) for m in range(0, batch, points)]
+            assert sum(runs) == batch and max(runs) * per_point * threads < 2 ** 32
+            split += len(runs) > 1
+    assert split > 0
