@@ -164,7 +164,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
         const OpacitySpecies& sp = species_[s];
         n = atm.nd(l, sp.species_id);                                 // opacity_species.cpp:407-412
         for (int q : sp.cia_partners) n *= atm.nd(l, q);
-        if (n != 0) ++lev[l].absorbers;
+        if (n > 0) ++lev[l].absorbers;
         if (groups.grouped) {
           // same grid as the group's representative: same bracket, own rows
           st = group_st[(groups.group1 >> s) & 1u];

@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
   }
   __syncthreads();
   // from here z holds two words per level: the slots whose rows changed (bit
-  // per slot) and the number of slots of non-zero density
+  // per slot) and the number of slots of positive density
   uint32_t* words = reinterpret_cast<uint32_t*>(z);
   for (int l = tid; l < 2 * L; l += kStageBlock) words[l] = 0;
   __syncthreads();
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       for (int k = 0; k < 4; ++k) block[k] = uint32_t(row[k] * P.blocks_per_row);
     }
     if (changed && s < 32) atomicOr(&words[2 * l], 1u << s);
-    if (dens != 0) atomicAdd(&words[2 * l + 1], 1u);
+    if (dens > 0) atomicAdd(&words[2 * l + 1], 1u);
     if (wide) {
       LevelSpecies& d = reinterpret_cast<LevelSpecies*>(rec + rec_species)[e];
       d.w[0] = (1.0 - ft) * (1.0 - fl) * kLog2Ten;
