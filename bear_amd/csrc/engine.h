@@ -42,10 +42,9 @@ struct Extras {
 // decides and the loads issue together.  What the forward kernels read comes
 // first, in whole lines of the scalar cache.
 struct alignas(64) LevelState {
-  double inv_temperature;
-  // half the thickness of the layer below this level; 0 at level 0, and, in a
-  // model without the H- continuum, where neither level holds a tabulated
-  // absorber (no opacity: an exact 0; with H-, withHminus sees to it)
+  double inv_temperature;    // of the level's Planck function (TabulatedModel::joinTransparentLayers)
+  // half the thickness of the layer below this level; 0 at level 0, and where
+  // neither level holds an absorbing gas (no opacity: an exact 0)
   double half_dz;
   double altitude;
   double rayleigh_density;   // number density of the Rayleigh scatterer (transmission)
@@ -322,6 +321,7 @@ class DeviceEngine {
   // the direct models' caller-given layer optical depths [levels - 1][N]
   // for the next evaluations (FixedCloudModel); NULL or all zero: none
   void setFixedCloud(const double* tau);
+  bool fixedCloudLayer(size_t level) const { return fixed_cloud_ && fixed_cloud_layers_[level]; }   // below `level`
   void uploadObservations(const std::vector<ObservationSetup>& observations);
   void configure(size_t nb_levels, size_t nb_species, bool transmission);
   void setStencilGroups(StencilGroups g) { groups_ = g; }
@@ -481,6 +481,7 @@ class DeviceEngine {
   CloudSpec cloud_spec_;
   double* cloud_tau_ = nullptr;                  // [L-1][N] caller-given cloud optical depths
   bool fixed_cloud_ = false;
+  std::vector<char> fixed_cloud_layers_;        // per level: any depth in the layer below it
   Extras extras() const { return Extras{hminus_, fixed_cloud_ ? cloud_tau_ : nullptr, cloud_spec_}; }
   double* flux_ = nullptr;
   double* spectrum_ = nullptr;

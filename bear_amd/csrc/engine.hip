@@ -550,6 +550,11 @@ void DeviceEngine::setFixedCloud(const double* tau) {
   bool any = false;                               // emission.cpp:344-360: an all-zero cloud is no cloud
   for (size_t i = 0; i < count && !any; ++i) any = tau[i] > 0;
   if (!any) return;
+  fixed_cloud_layers_.assign(nb_levels_, 0);
+  for (size_t l = 1; l < nb_levels_; ++l) {
+    const double* layer = tau + (l - 1) * n_points_;
+    fixed_cloud_layers_[l] = std::any_of(layer, layer + n_points_, [](double t) { return t != 0; });
+  }
   check(hipSetDevice(device_), "hipSetDevice");
   if (!cloud_tau_) cloud_tau_ = deviceAlloc<double>(count, "cloud optical depths");
   hipStream_t s = static_cast<hipStream_t>(stream_);

@@ -115,6 +115,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
   const double log2_ten = 3.321928094887362347870319429489390175864831393;
   const size_t blocks_per_row = engine_.tableStride() / 64;     // row -> block offset of the device tables
   const StencilGroups groups = engine_.stencilGroups();
+  bool absorbs = false;                                         // any gas of this level
   for (size_t l = 0; l < L; ++l) {
     Stencil group_st[2] = {};
     const double t = atm.temperature[l];
@@ -130,9 +131,10 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       lev[l].cloud_scale = transmission_ ? 1.0 / (atm.altitude[l] - atm.altitude[l - 1]) : 1.0;
       lev[l].half_dz = (atm.altitude[l] - atm.altitude[l - 1]) * 0.5;
     }
-    if (hminus_)                                    // H-, H and electron densities
-      hminusCoefficients(t, atm.nd(l, hminus_ids_[0]), atm.nd(l, hminus_ids_[1]), atm.nd(l, hminus_ids_[2]),
-                         lev[l].hminus_c);
+    const bool below_absorbs = absorbs;
+    absorbs = hminus_ &&                            // H-, H and electron densities
+              hminusCoefficients(t, atm.nd(l, hminus_ids_[0]), atm.nd(l, hminus_ids_[1]), atm.nd(l, hminus_ids_[2]),
+                                 lev[l].hminus_c);
     for (int g = 0; g < 2; ++g) {
       if (group_rep_[g] < 0) continue;
       const Stencil st = species_[size_t(group_rep_[g])].bracketLevel(l, t);
@@ -221,7 +223,8 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       }
       lev[l].reload |= changed << s;
     }
-    if (l > 0 && !hminus_ && lev[l].absorbers == 0 && lev[l - 1].absorbers == 0) lev[l].half_dz = 0.0;
+    absorbs = absorbs || lev[l].absorbers != 0;
+    if (l > 0 && !absorbs && !below_absorbs) lev[l].half_dz = 0.0;
   }
   size_t k = 0;                                                   // forward_model.cpp:184-204
   for (size_t o = 0; o < observations_.size(); ++o) {
@@ -230,11 +233,30 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
   }
 }
 
+// A layer without any absorption passes the intensity on unchanged, so above
+// the lowest level of a run of such layers no level's Planck function enters
+// the flux, but the uppermost one's where an absorbing layer follows.  Those
+// levels take the lowest one's: the sweeps sum differences of Planck functions
+// (emission_sweep.h), which are exact zeros then.  Left alone, hot transparent
+// levels over a cold atmosphere, larger by up to 1e30 at visible wavelengths,
+// would have to cancel.
+void TabulatedModel::joinTransparentLayers(LevelState* lev) const {
+  const size_t L = atmosphere_.nb_levels;
+  auto transparent = [&](size_t l) {                             // the layer below level l
+    bool clear = lev[l].half_dz == 0 && !engine_.fixedCloudLayer(l);
+    for (double w : lev[l].cloud_w) clear = clear && w == 0;
+    return clear;
+  };
+  for (size_t l = 1; l < L; ++l)
+    if (transparent(l) && (l + 1 == L || transparent(l + 1))) lev[l].inv_temperature = lev[l - 1].inv_temperature;
+}
+
 void TabulatedModel::stageStructure(double g, double radius, bool variable_gravity, const double* p, const double* t,
                                     const std::vector<int>& species, const double* x) {
   atmosphere_.setStructure(g, radius, variable_gravity, p, t, species, x);
   for (OpacitySpecies& s : species_) s.preparePressures(atmosphere_.pressure);   // this call's pressures
   stageLevels(atmosphere_, nullptr, engine_.levels(), engine_.levelSpecies(), nullptr, nullptr, engine_.shifts());
+  joinTransparentLayers(engine_.levels());
 }
 
 bool TabulatedModel::stage(const double* p, BatchModel& scalars) {
@@ -244,6 +266,7 @@ bool TabulatedModel::stage(const double* p, BatchModel& scalars) {
               engine_.shifts());
   CloudSpec spec;
   if (!clouds_.empty()) stageClouds(atmosphere_, clouds(p), std::pow(10, p[0]), fixedScaleHeight(p), engine_.levels(), spec);
+  joinTransparentLayers(engine_.levels());
   engine_.setCloudSpec(spec);
   return neglect;
 }
@@ -344,6 +367,7 @@ void TabulatedModel::stageBatch(const double* params, size_t batch, size_t strid
                   engine_.batchShifts(b));
       if (!clouds_.empty())
         stageClouds(atm, clouds(p), std::pow(10, p[0]), fixedScaleHeight(p), engine_.batchLevels(b), scalars.clouds);
+      joinTransparentLayers(engine_.batchLevels(b));
     } catch (const Error& e) {
 #pragma omp critical(bear_stage_failure)
       if (failure.empty()) { failure = e.what(); failure_code = e.code; }

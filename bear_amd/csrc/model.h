@@ -130,6 +130,7 @@ class TabulatedModel : public ForwardModel {
   // H- continuum's weights also give temperature terms, added to t_bar)
   void densityGradient(const Atmosphere& atm, const double* G, std::vector<double>& n_bar,
                        std::vector<double>& t_bar) const;
+  void joinTransparentLayers(LevelState* levels) const;     // the staged levels, clouds included
   size_t cloudSlot() const { return adjointCloudSlot(engine_.speciesStride(), hminus_); }
   size_t levelSlots() const { return adjointSlots(engine_.speciesStride(), hminus_, !clouds_.empty()); }
   // d logL / d the cloud models' optical depths and spectral parameters

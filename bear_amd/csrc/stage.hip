@@ -407,10 +407,19 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
     }
   }
   __syncthreads();
+  // the layer below level l is transparent (no clouds and no H- here)
+  auto transparent = [&](int l) { return l > 0 && words[2 * l + 1] == 0 && words[2 * l - 1] == 0; };
   for (int l = tid; l < L; l += kStageBlock) {
     lev[l].reload = words[2 * l];
     lev[l].absorbers = words[2 * l + 1];
-    if (l > 0 && words[2 * l + 1] == 0 && words[2 * l - 1] == 0) lev[l].half_dz = 0.0;
+    if (transparent(l)) {
+      lev[l].half_dz = 0.0;
+      if (l + 1 == L || transparent(l + 1)) {         // TabulatedModel::joinTransparentLayers
+        int lowest = l;
+        while (transparent(lowest)) --lowest;
+        lev[l].inv_temperature = lev[lowest].inv_temperature;
+      }
+    }
   }
 }
 
