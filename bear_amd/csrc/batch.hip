@@ -380,8 +380,11 @@ void DeviceEngine::launchBatchRest(ModelKind kind, size_t batch, size_t first) {
   }
 }
 
-// Autotuner: times the spectrum kernel of the first min(batch, 64) staged
-// points for each candidate launch shape and keeps the fastest.
+// Autotuner: times the spectrum kernel for each candidate launch shape and
+// keeps the fastest, on the records that the host holds of the first
+// min(batch, 64) points.  A batch staged on the device leaves those as they
+// were, all zeros at first: the kernels then do their full work on values that
+// mean nothing, without the early ends of opaque columns and paths.
 //   emission / eclipse: workgroups of 128 or 256 wavenumbers; where that
 //     leaves the chip under four rounds of wavefronts, also tiles of 64
 //     wavenumbers with their levels split over 2, 4 or 8 wavefronts
@@ -408,13 +411,16 @@ BatchLaunch DeviceEngine::tune(ModelKind kind, size_t batch) {
       const size_t items = nbItems(int((n_points_ + tile - 1) / tile), int(batch));
       return BatchLaunch{block, tile, int(std::min<size_t>(items, INT32_MAX)), kPointGroup, split};
     };
+    const size_t tiles = (n_points_ + 63) / 64 * batch;
+    const int split = levelSplit(tiles, nb_cus_);
+    if (!autotune_) return split > 1 ? shape(64 * split, 64, split) : shape(256, 256, 1);
     for (int block : {256, 128}) cand.push_back(shape(block, block, 1));
-    if ((n_points_ + 63) / 64 * batch < size_t(nb_cus_) * 64)
-      for (int split : {2, 4, 8}) cand.push_back(shape(64 * split, 64, split));
+    if (tiles < size_t(nb_cus_) * 64)
+      for (int k : {2, 4, 8}) cand.push_back(shape(64 * k, 64, k));
   }
   if (kind == ModelKind::transmission)
     for (auto& c : cand) c.grid = int(align(size_t(c.grid), 8));
-  if (!autotune_) return kind == ModelKind::transmission ? cand[cand.size() / 2] : cand.front();
+  if (!autotune_) return cand[cand.size() / 2];
   check(hipMemcpyAsync(batch_dev_, batch_host_, b * rec_bytes_, hipMemcpyHostToDevice, s), "upload batch");
   hipEvent_t e0, e1;
   check(hipEventCreate(&e0), "hipEventCreate");

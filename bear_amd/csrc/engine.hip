@@ -714,16 +714,11 @@ void DeviceEngine::launchBins(int mode, double star_temperature, double depth_sc
 namespace {
 bool hasExtras(const Extras& ex) { return ex.hminus || ex.cloud_tau || ex.clouds.count > 0; }
 
-// Wavefronts that share one tile's levels: 8 up to 8 tiles per CU, 4 up to 16
-// per CU (4,096 tiles, 262,144 wavenumbers), so that a launch has 8 to 64
-// wavefronts per CU, else 1.  Beyond, whole columns are the faster.
-int levelSplit(int tiles, int cus) { return tiles <= cus * 8 ? 8 : tiles <= cus * 16 ? 4 : 1; }
-
 void launchEmission(hipStream_t s, size_t species_stride, int cus, const double* nu, const double* lam,
                     const double* tables, size_t stride, const Extras& ex, const LevelState* lev,
                     const LevelSpecies* spc, StencilGroups groups, int L, int n, double min_inv_t, double scaling,
                     SpectrumOut out, double* flux, double* spectrum) {
-  const int tiles = (n + 63) / 64, split = levelSplit(tiles, cus);
+  const int tiles = (n + 63) / 64, split = levelSplit(size_t(tiles), cus);
   const dim3 grid{unsigned(split > 1 ? tiles : (n + kBlock - 1) / kBlock)},
       block{unsigned(split > 1 ? 64 * split : kBlock)};
   const size_t lds = split > 1 ? splitPart(split) * sizeof(double) : 0;

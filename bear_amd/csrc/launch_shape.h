@@ -55,6 +55,19 @@ constexpr TransitShape transitShape(int levels, size_t slots, bool isothermal, s
   return {false, kTransitThreads, tile, 0, sums};
 }
 
+// Emission: wavefronts that share one tile's levels, by the tiles of a launch:
+// 8 up to 8 tiles per CU, 4 up to 16, so that it has 8 to 64 wavefronts per CU,
+// else 1, whole columns, which stop where they are opaque.  One point of 100
+// levels and 8 slots, us per likelihood in 1 / 2 / 4 / 8 wavefronts per tile:
+//    0.7 tiles per CU  187 / 120 /  86 /  72     17.8  321 / 382 / 256 / 270
+//    5.9               193 / 205 / 132 / 127     29.7  431 / 562 / 388 / 415
+//   11.9               241 / 290 / 191 / 198     47.4  608 / 828 / 586 / 642
+// (above 16 per CU 4 wavefronts would still gain 4 to 20 % there; with 14 slots
+// 23.7 per CU take 657 / 706 / 663 / 751, with 17.8 634 / 531 / 512 / 583).
+constexpr int levelSplit(size_t tiles, int cus) {
+  return tiles <= size_t(cus) * 8 ? 8 : tiles <= size_t(cus) * 16 ? 4 : 1;
+}
+
 // A launch takes fewer than 2^32 threads in x.  Workgroups at most, in whole
 // rounds of the 8 XCDs (device_math.h, workItem).
 constexpr size_t maxWorkgroups(int threads) { return ((size_t(1) << 32) - 1) / size_t(threads) / 8 * 8; }

@@ -80,3 +80,16 @@ def test_launches_of_large_batches(tmp_path):
             assert sum(runs) == batch and max(runs) * per_point * threads < 2 ** 32
             split += len(runs) > 1
     assert split > 0
+
+
+def test_level_split_by_tiles(tmp_path):
+    """Eight wavefronts per tile, then four, then one, and never fewer than
+    eight wavefronts per CU where the split could give them."""
+    cus = 256
+    rows = _run(str(tmp_path), """
+  for (size_t tiles = 1; tiles <= 8 * %d * 4; ++tiles) std::printf("%%zu %%d\\n", tiles, levelSplit(tiles, %d));
+""" % (cus, cus))
+    splits = [s for _, s in rows]
+    assert set(splits) == {8, 4, 1} and splits == sorted(splits, reverse=True)
+    assert all(tiles * split >= 8 * cus for tiles, split in rows if tiles >= cus)
+    assert splits[8 * cus - 1] == 8 and splits[8 * cus] == 4 and splits[16 * cus - 1] == 4 and splits[16 * cus] == 1
