@@ -1160,8 +1160,12 @@ void DeviceEngine::evaluateAdjointBatch(ModelKind kind, size_t batch, std::vecto
     raise(kInvalidInput, "the H- continuum's gradient needs the kept forward quantities: raise the adjoint memory");
   if (cloud_models_ > 0 && !kept)
     raise(kInvalidInput, "the clouds' gradient needs the kept forward quantities: raise the adjoint memory");
-  // the emission forward runs in workgroups of 256, the transmission forward
-  // as tuned
+  // the transmission forward runs as tuned, the emission forward in workgroups
+  // of 256: per gradient call in workgroups of 64 / 128 / 256, us
+  //    2,373 wavenumbers,  40 levels,  4 slots,  1 point     232 /  236 /  238
+  //    2,373              100         14         4 points    583 /  601 /  609
+  //   18,974              100          8        16          1161 / 1074 / 1077
+  //   85,381              100          8        32          6865 / 6398 / 6507
   const BatchLaunch launch = !transmission ? BatchLaunch{256, 256, int(std::min<size_t>(nbItems((n + 255) / 256, int(chunk)), INT32_MAX))}
                                                    : tuned(kind, chunk);
   last_launch_ = launch;

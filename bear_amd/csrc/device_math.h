@@ -132,7 +132,11 @@ __device__ __forceinline__ void starFluxWithDerivative(double nu, double inv_t, 
 // kept in registers between levels and all reloaded when the level brings new
 // rows for some slot (opacity_species.cpp:277-345, 400-433: the bilinear log10
 // interpolation in T and log p, times the effective density).  Rows are always
-// valid; a zero density (kZeroDensityLog2) removes a term exactly.
+// valid; a zero density (kZeroDensityLog2) removes a term exactly here, and in
+// the reduced-precision opacity; the forms over the LDS table (opacity64.h)
+// keep a term of at most 2^-340 sigma, far below the last bit of any other, so
+// that where nothing else absorbs a layer's zero has to be seen to by itself
+// (LevelState::half_dz, withHminus).
 // With grouped stencils (StencilGroups) the weights come from the level's two
 // shared sets and the densities from the level's contiguous copy (NS <= 16);
 // otherwise both from each slot's record.

@@ -1,4 +1,6 @@
-// FP64 powers of two from a table in LDS.
+// FP64 powers of two from a table in LDS: a table of the octave's steps and a
+// short polynomial within a step (P. T. P. Tang, Table-driven implementation of
+// the exponential function, ACM TOMS 15, 1989).
 //
 // 2^(i / 128 + f / 128) = 2^(i / 128) P(f): the table holds 2^(j / 128) for j
 // in [0, 128), and P is a polynomial of degree 3 or 4 in f, so that a power
