@@ -35,7 +35,8 @@ SPECTRUM_BAR = 1e-5         # relative, emission spectra and bins
 LOGLIKE_BAR = 1e-6          # absolute
 # the sources of the single-point kernel: a counter profile is valid for these only
 KERNEL_SOURCES = ("bear_amd/csrc/engine.hip", "bear_amd/csrc/device_math.h", "bear_amd/csrc/engine.h",
-                  "bear_amd/csrc/emission_sweep.h", "bear_amd/csrc/exp_table.h", "bear_amd/csrc/opacity64.h")
+                  "bear_amd/csrc/emission_sweep.h", "bear_amd/csrc/exp_table.h", "bear_amd/csrc/opacity64.h",
+                  "bear_amd/csrc/launch_shape.h")
 
 
 def log(msg):
