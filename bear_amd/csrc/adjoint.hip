@@ -27,7 +27,7 @@
 // The kernels over kept quantities take one work item per workgroup of one
 // wavefront, levelled by the dispatcher: 32 points of 100 levels, 8 species
 // and 50,000 wavenumbers 5.00 -> 4.46 ms per gradient call against persistent
-// grids of 16 wavefronts per CU.  FP64 issue bounds them (70 to 76 % busy).
+// grids of 16 wavefronts per CU.  FP64 issue bounds them (64 and 83 % busy).
 // When one point's kept quantities exceed the budget, emissionAdjointKernel
 // does all of it for each work item, recomputing its forward sweep into a
 // per-workgroup scratch first.
