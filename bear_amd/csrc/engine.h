@@ -49,7 +49,7 @@ struct alignas(64) LevelState {
   double altitude;
   double rayleigh_density;   // number density of the Rayleigh scatterer (transmission)
   uint32_t reload;           // bit s: slot s's rows changed
-  uint32_t absorbers;        // slots of positive density (any other counts as zero)
+  uint32_t absorbers;        // slots whose density is not zero or negative (which counts as zero)
   // a layer's cloud optical depth as this level's term: 1 for emission,
   // 1 / (z_l - z_{l-1}) for transmission (an extinction, cloud_model.h:67-88)
   double cloud_scale;

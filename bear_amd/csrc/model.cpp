@@ -166,7 +166,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
         const OpacitySpecies& sp = species_[s];
         n = atm.nd(l, sp.species_id);                                 // opacity_species.cpp:407-412
         for (int q : sp.cia_partners) n *= atm.nd(l, q);
-        if (n > 0) ++lev[l].absorbers;
+        if (!(n <= 0)) ++lev[l].absorbers;
         if (groups.grouped) {
           // same grid as the group's representative: same bracket, own rows
           st = group_st[(groups.group1 >> s) & 1u];
@@ -224,7 +224,7 @@ void TabulatedModel::stageLevels(const Atmosphere& atm, const double* mods, Leve
       lev[l].reload |= changed << s;
     }
     absorbs = absorbs || lev[l].absorbers != 0;
-    if (l > 0 && !absorbs && !below_absorbs) lev[l].half_dz = 0.0;
+    if (l > 0 && !absorbs && !below_absorbs) lev[l].half_dz *= 0.0;       // a NaN thickness stays
   }
   size_t k = 0;                                                   // forward_model.cpp:184-204
   for (size_t o = 0; o < observations_.size(); ++o) {

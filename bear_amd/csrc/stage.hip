@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
   }
   __syncthreads();
   // from here z holds two words per level: the slots whose rows changed (bit
-  // per slot) and the number of slots of positive density
+  // per slot) and the number of slots that can absorb (LevelState::absorbers)
   uint32_t* words = reinterpret_cast<uint32_t*>(z);
   for (int l = tid; l < 2 * L; l += kStageBlock) words[l] = 0;
   __syncthreads();
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
       for (int k = 0; k < 4; ++k) block[k] = uint32_t(row[k] * P.blocks_per_row);
     }
     if (changed && s < 32) atomicOr(&words[2 * l], 1u << s);
-    if (dens > 0) atomicAdd(&words[2 * l + 1], 1u);
+    if (!(dens <= 0)) atomicAdd(&words[2 * l + 1], 1u);
     if (wide) {
       LevelSpecies& d = reinterpret_cast<LevelSpecies*>(rec + rec_species)[e];
       d.w[0] = (1.0 - ft) * (1.0 - fl) * kLog2Ten;
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kStageBlock) void stageKernel(StagePlan P, const un
     lev[l].reload = words[2 * l];
     lev[l].absorbers = words[2 * l + 1];
     if (transparent(l)) {
-      lev[l].half_dz = 0.0;
+      lev[l].half_dz *= 0.0;                          // a NaN thickness stays
       if (l + 1 == L || transparent(l + 1)) {         // TabulatedModel::joinTransparentLayers
         int lowest = l;
         while (transparent(lowest)) --lowest;
